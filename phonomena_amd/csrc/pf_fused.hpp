@@ -433,7 +433,7 @@ inline TileMap fused_map(const pf_ctx* c, int tj, int kz, int xchunk, long long 
     tm.nkt = (c->nz + (kz - 4) - 1) / (kz - 4);
     tm.njt = (c->ny + (tj - 4) - 1) / (tj - 4);
     if (xchunk <= 0 && slots > 0) {
-        xchunk = round_xchunk((long long)tm.nkt * tm.njt, c->nx, 3, 32, XT2 - 6, slots);
+        xchunk = round_xchunk((long long)tm.nkt * tm.njt, c->nx, 3, 0, 32, XT2 - 6, slots);
     } else if (xchunk <= 0) {
         // aim for ~1024 blocks (4 per CU) with chunks of at least 32 planes
         const long long per = (long long)tm.nkt * tm.njt;

@@ -38,6 +38,13 @@ struct pf_ctx {
     int precision = 0, kernel = 0, tile_j = 4, tile_x = 0, tile_z = 64;
     int pair_j = 0, pair_z = 0;  // tile of the two-step sweep (PF_KERNEL_TILED2)
     bool shape_open = false;     // tile shape left to measurement at creation
+    // planes per x chunk of the one-step sweep, for the shape and resident
+    // blocks it was last chosen for (tile_map)
+    mutable struct {
+        int tj = 0, kz = 0;
+        long long slots = 0;
+        int xchunk = 0;
+    } auto_chunk;
     size_t esz = 8;
     bool sponge = false;
     int surface = 0;  // pf_desc.surface

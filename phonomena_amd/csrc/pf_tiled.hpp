@@ -558,13 +558,21 @@ template <class K> int blocks_per_cu(K kernel, int threads) {
 
 // Planes per x chunk, from the rounds in which the device runs the blocks.
 // per tiles per plane, each block marching xc planes plus `warm` planes it
-// only loads and computes; `slots` blocks resident at once.  Over the
-// balanced chunkings (n chunks of ceil(nx / n) planes, lo <= planes <= cap)
-// the one with the most useful planes per resident-block plane time:
-//     per * nx / (slots * rounds * (xc + warm)),  rounds = ceil(per * n / slots)
+// only loads and computes, in pairs, after a start that costs about `start`
+// planes; `slots` blocks resident at once.  Over the balanced chunkings (n
+// chunks of ceil(nx / n) planes, lo <= planes <= cap) the one with the most
+// useful planes per resident-block plane time:
+//     per * nx / (slots * rounds * (even(xc + warm) + start)),
+//     rounds = ceil(per * n / slots)
 // which charges a last round that leaves CUs idle and the warm-up planes
-// of short chunks.  Ties go to more chunks.
-inline int round_xchunk(long long per, int nx, int warm, int lo, int cap, long long slots) {
+// of short chunks.  Ties go to more chunks.  The one-step sweep takes chunks
+// down to 2 planes: where a launch is one round (meshes under about a
+// million nodes) its time is the planes a block marches one after another
+// (0.7 us each in FP32, 1.6 us in FP64 with divisions).  Measured against
+// chunks of at least 16 planes, microseconds a step: 65 x 65 x 33 nodes FP32
+// 12.7 / 22.8, FP32C 18.1 / 37.5, FP64 18.9 / 39.4; 58 x 39 x 13 FP64 15.8 /
+// 45.5; 129 x 129 x 65 FP32 21.3 / 25.9, FP32C 34.4 / 41.4.
+inline int round_xchunk(long long per, int nx, int warm, int start, int lo, int cap, long long slots) {
     int best = nx < cap ? nx : cap;
     double best_s = -1.0;
     for (int n = 1; n <= nx; n++) {
@@ -575,7 +583,8 @@ inline int round_xchunk(long long per, int nx, int warm, int lo, int cap, long l
         if (nc != n) continue;  // same chunking as a smaller n
         const long long blocks = per * nc;
         const long long rounds = (blocks + slots - 1) / slots;
-        const double sc = (double)per * nx / ((double)slots * (double)rounds * (double)(xc + warm));
+        const int planes = (xc + warm + 1) / 2 * 2 + start;
+        const double sc = (double)per * nx / ((double)slots * (double)rounds * (double)planes);
         if (sc >= best_s) {
             best_s = sc;
             best = xc;
@@ -591,7 +600,11 @@ inline TileMap tile_map(const pf_ctx* c, int tj, int kz, int xchunk, long long s
     tm.nkt = (c->nz + (kz - 2) - 1) / (kz - 2);
     tm.njt = (c->ny + (tj - 2) - 1) / (tj - 2);
     if (xchunk <= 0 && slots > 0) {
-        xchunk = round_xchunk((long long)tm.nkt * tm.njt, c->nx, 1, 16, XT - 3, slots);
+        // chosen once per shape: the search costs as much host time as a launch
+        auto& a = c->auto_chunk;
+        if (a.tj != tj || a.kz != kz || a.slots != slots)
+            a = {tj, kz, slots, round_xchunk((long long)tm.nkt * tm.njt, c->nx, 1, 2, 2, XT - 3, slots)};
+        xchunk = a.xchunk;
     } else if (xchunk <= 0) {
         // aim for >= ~2048 blocks (8 per CU) with chunks of at least 16 planes
         const long long per = (long long)tm.nkt * tm.njt;
