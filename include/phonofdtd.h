@@ -42,7 +42,10 @@ extern "C" {
 
 /* Sweep kernel.  PF_KERNEL_AUTO: PF_KERNEL_TILED2 for PF_FP32 meshes of at
    least PF_TILED2_AUTO_NODES nodes (>= 8 per axis), else PF_KERNEL_TILED;
-   PF_KERNEL_NAIVE beyond 16 materials or a 4 GiB time level. */
+   PF_KERNEL_NAIVE beyond 16 materials or a 4 GiB time level.  With AUTO and
+   no tile fields, meshes of up to about 10^5 nodes take whole steps in
+   blocks instead of marching tiles, several steps a launch (the same bits;
+   pf_kernel_info reports PF_KERNEL_TILED and its fixed shape). */
 #define PF_KERNEL_AUTO 0
 #define PF_TILED2_AUTO_NODES (1LL << 24)
 #define PF_KERNEL_NAIVE 1   /* one thread per node, stresses recomputed     */

@@ -18,6 +18,7 @@
 #include "pf_fused.hpp"
 #include "pf_raster.hpp"
 #include "pf_tiled.hpp"
+#include "pf_block.hpp"
 
 using namespace pf;
 
@@ -149,9 +150,6 @@ template <class R>
 static int create_tables(pf_ctx* c, const pf_desc* d) {
     const bool exact = d->precision == PF_FP64;
     int rc;
-    // the FP64 one-step tiled sweep on power-of-two spacings multiplies by
-    // exact reciprocals (MODE_FP64P)
-    c->recip = exact && c->kernel == PF_KERNEL_TILED && pow2_spacings(d);
     if (c->recip) {
         if ((rc = upload_table(&c->rfx, spacing_table<double>(d->fdx, d->nx - 1, true)))) return rc;
         if ((rc = upload_table(&c->rfy, spacing_table<double>(d->fdy, d->ny - 1, true)))) return rc;
@@ -234,6 +232,27 @@ static int rasterize(pf_ctx* c, const pf_desc* d) {
     } while (0);
     cleanup();
     return rc;
+}
+
+// Whether a context of the one-step tiled sweep steps in blocks instead, and
+// with how many steps a launch: the cheapest by block_map's estimate, if that
+// is below what the march takes at the least.
+static void block_plan(pf_ctx* c) {
+    if (c->cells > BLOCK_MAX_CELLS || c->cus < 1) return;
+    const BlockCost cost = block_cost(c->precision == PF_FP64   ? (c->recip ? MODE_FP64P : MODE_FP64)
+                                      : c->precision == PF_FP32 ? MODE_FP32
+                                                                : MODE_FP32C);
+    double best = cost.march;
+    for (int r = 1; r <= BLOCK_MAX_STEPS; r++) {
+        double us = 0;
+        c->block[r] = block_map(c->nx, c->ny, c->nz, r, c->cus, cost, &us);
+        if (c->block[r].threads == 0) break;
+        if (us / r < best) {
+            best = us / r;
+            c->block_steps = r;
+        }
+    }
+    if (c->block_steps) c->shape_open = false;
 }
 
 int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
@@ -339,6 +358,10 @@ int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
         (void)hipGetLastError();
         c->cus = 0;
     }
+    // the FP64 one-step tiled sweep and block steps on power-of-two spacings
+    // multiply by exact reciprocals (MODE_FP64P)
+    c->recip = d->precision == PF_FP64 && c->kernel == PF_KERNEL_TILED && pow2_spacings(d);
+    if (d->kernel == PF_KERNEL_AUTO && c->kernel == PF_KERNEL_TILED && c->shape_open && c->tile_x == 0) block_plan(c);
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
 
     // fields: two levels (four for the two-step sweep) x three components
@@ -355,7 +378,7 @@ int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
     const size_t bytes = (size_t)c->cells * c->esz;
     const size_t lbytes = (size_t)c->cells * sizeof(lo_t);
     const size_t lvl_bytes = level_bytes(c->cells, c->precision);
-    c->nlevels = pair ? 4 : 2;
+    c->nlevels = pair || c->block_steps ? 4 : 2;
     for (int l = 0; l < c->nlevels; l++) {
         HIPCHK(hipMalloc(&c->lvlbase[l], lvl_bytes + (size_t)l * PF_LEVEL_STAGGER));
         char* b = (char*)c->lvlbase[l] + (size_t)l * PF_LEVEL_STAGGER;
@@ -762,6 +785,58 @@ int pf::step_once(pf_ctx* c, hipStream_t s, const long long* base, long long off
     }
 }
 
+// r steps of a small mesh in one launch (pf_block.hpp): for one step the new
+// level goes over the previous one, for more the last two levels go to the
+// two buffers not in use.
+template <class R, int MODE>
+static int step_block_t(pf_ctx* c, hipStream_t s, long long off, int r, hipEvent_t* ev) {
+    int a1 = c->old, a2 = c->cur;
+    if (r > 1) {
+        a1 = a2 = -1;
+        for (int l = 0; l < c->nlevels; l++)
+            if (l != c->cur && l != c->old) (a1 < 0 ? a1 : a2) = l;
+        if (a2 < 0) return fail(PF_ERR_STATE, "block steps without their level buffers");
+    }
+    Mesh<R> m = sweep_view<R, MODE>(c, c->cur, c->old, a1);
+    m.step_off = off;
+    R* p[3];
+    lo_t* pl[3];
+    for (int q = 0; q < 3; q++) {
+        p[q] = (R*)c->lvl[a2][q];
+        pl[q] = (lo_t*)c->lvlo[a2][q];
+    }
+    FaceProbe pr = {};
+    pr.every = 1;
+    if (c->probe[2] > 0 && (off + r) / c->every > off / c->every) {  // a step among them records
+        const int* q = c->probe;
+        pr = {c->ring, c->d_frame, (int*)(c->d_frame + 1), q[0], q[1], q[2], q[3], q[4], q[5], c->cap, c->every, 0};
+    }
+    if (ev) HIPCHK(hipEventRecord(ev[0], s));
+    const int rc = c->sponge ? launch_block_k<R, MODE, true>(m, c->block[r], p, pl, pr, s)
+                             : launch_block_k<R, MODE, false>(m, c->block[r], p, pl, pr, s);
+    if (rc) return rc;
+    if (ev) HIPCHK(hipEventRecord(ev[1], s));
+    if (r == 1) {
+        const int t = c->cur;
+        c->cur = c->old;
+        c->old = t;
+    } else {
+        c->cur = a1;
+        c->old = a2;
+    }
+    return PF_OK;
+}
+
+static int step_block(pf_ctx* c, hipStream_t s, long long off, int r, hipEvent_t* ev) {
+    switch (c->precision) {
+        case PF_FP64:
+            return c->recip ? step_block_t<double, MODE_FP64P>(c, s, off, r, ev)
+                            : step_block_t<double, MODE_FP64>(c, s, off, r, ev);
+        case PF_FP32: return step_block_t<float, MODE_FP32>(c, s, off, r, ev);
+        default: return step_block_t<float, MODE_FP32C>(c, s, off, r, ev);
+    }
+}
+
 extern "C" int pf_step(pf_ctx* c, int64_t nsteps) {
     if (!c) return fail(PF_ERR_ARG, "ctx is NULL");
     if (c->batch) return fail(PF_ERR_STATE, "context is stepped by its batch");
@@ -770,6 +845,13 @@ extern "C" int pf_step(pf_ctx* c, int64_t nsteps) {
         return fail(PF_ERR_RANGE, "step %lld + %lld beyond the source table (%lld)", (long long)c->step,
                     (long long)nsteps, (long long)c->wave_len);
     int64_t s = 0;
+    while (c->block_steps && s < nsteps) {
+        const int r = (int)(nsteps - s < c->block_steps ? nsteps - s : c->block_steps);
+        int rc = step_block(c, c->stream, c->step, r, nullptr);
+        if (rc) return rc;
+        c->step += r;
+        s += r;
+    }
     if (c->kernel == PF_KERNEL_TILED2) {
         for (; s + 2 <= nsteps; s += 2) {
             int rc = step_pair(c, c->stream, nullptr, c->step, nullptr);
@@ -1121,8 +1203,9 @@ extern "C" int pf_profile(pf_ctx* c, int64_t nsteps, double* sweep_ms, double* f
     // the rest (faces, probes, the band of a pair, launch gaps) = the span
     // from the first event to the last less the sweeps.  The events are the
     // context's own, created by the first call.
-    const int64_t pairs = c->kernel == PF_KERNEL_TILED2 ? nsteps / 2 : 0;
-    const int64_t singles = nsteps - 2 * pairs;
+    const int64_t group = c->kernel == PF_KERNEL_TILED2 ? 2 : c->block_steps > 1 ? c->block_steps : 0;
+    const int64_t pairs = group ? nsteps / group : 0;
+    const int64_t singles = nsteps - group * pairs;
     auto stride_of = [](int64_t groups) {
         const int64_t s = (groups + PF_PROFILE_BRACKETS - 1) / PF_PROFILE_BRACKETS;
         return s > 4 ? s : (int64_t)4;
@@ -1144,14 +1227,15 @@ extern "C" int pf_profile(pf_ctx* c, int64_t nsteps, double* sweep_ms, double* f
     for (int64_t g = 0; g < pairs && !rc; g++) {
         hipEvent_t* e = g % pstride == 0 ? &ev[used] : nullptr;
         if (e) used += 2;
-        rc = step_pair(c, c->stream, nullptr, c->step, e);
-        if (!rc) c->step += 2;
+        rc = c->block_steps ? step_block(c, c->stream, c->step, (int)group, e)
+                            : step_pair(c, c->stream, nullptr, c->step, e);
+        if (!rc) c->step += group;
     }
     const size_t pair_ev = used;
     for (int64_t g = 0; g < singles && !rc; g++) {
         hipEvent_t* e = g % sstride == 0 ? &ev[used] : nullptr;
         if (e) used += 2;
-        rc = step_once(c, c->stream, nullptr, c->step, e);
+        rc = c->block_steps ? step_block(c, c->stream, c->step, 1, e) : step_once(c, c->stream, nullptr, c->step, e);
         if (!rc) c->step++;
     }
     if (!rc) {

@@ -24,11 +24,22 @@
 #define PF_PROFILE_BRACKETS 8
 #define PF_PROFILE_EVENTS (4 * PF_PROFILE_BRACKETS + 1)
 
+namespace pf {
+// A partition of the mesh into ntx x nty x ntz owned boxes (balanced; at
+// least 3 nodes an axis, so a box that holds a face holds the cells its Mur
+// map reads) for launches of `steps` whole steps, and the threads that the
+// largest box with its halo needs (pf_block.hpp).
+struct BlockMap {
+    int ntx, nty, ntz, steps, threads;
+};
+constexpr int BLOCK_MAX_STEPS = 4;
+}  // namespace pf
+
 // One mesh on one device.  Time levels of the displacement components are
 // kept in level buffers: `cur` indexes the current level (n) and `old` the
 // previous one (n-1); a single step overwrites `old` with level n+1 and
-// swaps the two.  Two-step sweeps use two more level buffers (allocated on
-// first use).  Each level is one allocation holding its arrays back to back
+// swaps the two.  Two-step sweeps and block steps use two more level
+// buffers.  Each level is one allocation holding its arrays back to back
 // (ux, uy, uz, then the 16-bit lo parts in FP32C), so one buffer descriptor
 // covers a whole level; level l starts l * PF_LEVEL_STAGGER bytes into its
 // allocation (lvlbase[l] is the allocation, lvl[l][0] the level).
@@ -45,6 +56,10 @@ struct pf_ctx {
         long long slots = 0;
         int xchunk = 0;
     } auto_chunk;
+    // a small mesh: whole steps in blocks, block_steps a launch at most, with
+    // the partition for r steps at block[r]
+    int block_steps = 0;
+    pf::BlockMap block[pf::BLOCK_MAX_STEPS + 1] = {};
     size_t esz = 8;
     bool sponge = false;
     int surface = 0;  // pf_desc.surface
