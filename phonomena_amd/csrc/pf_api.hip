@@ -455,9 +455,6 @@ int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
         HIPCHK(hipMalloc((void**)&c->d_frame, 2 * sizeof(long long)));
         HIPCHK(hipMemsetAsync(c->d_frame, 0, 2 * sizeof(long long), c->stream));
     }
-    HIPCHK(hipMalloc((void**)&c->e_out, 2 * sizeof(double)));
-    c->e_blocks = 1024;
-    HIPCHK(hipMalloc((void**)&c->e_partials, 2 * sizeof(double) * (size_t)c->e_blocks));
     // the clears above are ordered on the context's own stream; waiting for
     // it (not the whole device) lets a context be created while other
     // contexts' or a batch's work runs
@@ -474,7 +471,8 @@ void pf::ctx_free(pf_ctx* c) {
     F(c->rfx); F(c->rfy); F(c->rfz); F(c->rsx); F(c->rsy); F(c->rsz);
     F(c->dpx); F(c->dpy); F(c->dpz);
     F(c->mat64); F(c->rho64); F(c->fx64); F(c->fy64); F(c->fz64); F(c->sx64); F(c->sy64); F(c->sz64);
-    F(c->wave); F(c->d_step); F(c->ring); F(c->d_frame); F(c->e_out); F(c->e_partials);
+    F(c->wave); F(c->d_step); F(c->ring); F(c->d_frame); F(c->e_partials);
+    if (c->e_out) (void)hipHostFree(c->e_out);
     F(c->scratch);
     if (c->snap_stream) (void)hipStreamSynchronize(c->snap_stream);  // no copy in flight
     F(c->snap_dev);
@@ -1128,61 +1126,52 @@ extern "C" int pf_get_probes(pf_ctx* c, double* host, int64_t cap_frames, int64_
 }
 
 // ------------------------------------------------------------- energy ----
-template <class R>
-__global__ void k_widen(const R* __restrict__ hi, const lo_t* __restrict__ lo, double* __restrict__ out, long long n) {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const R h = hi[t];
-    double v = (double)h;
-    if (lo) v += (double)lo_decode(h, lo[t]);
-    out[t] = v;
+template <class R, bool COMP>
+static int launch_energy(pf_ctx* c, const EnergyArgs& ea, dim3 grid, hipStream_t s) {
+    const Mesh<R> m = make_view<R>(c, c->cur, c->old, c->old);
+    const size_t lds = (size_t)c->nmat * (MAT_STRIDE + 1) * sizeof(double);
+    const auto kernel = k_energy_partial<R, COMP>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, m, ea, c->e_partials);
+    HIPCHK(hipGetLastError());
+    return PF_OK;
 }
 
 extern "C" int pf_energy(pf_ctx* c, double* out) {
     if (!c || !out) return fail(PF_ERR_ARG, "NULL argument");
     hipStream_t s = c->batch ? c->batch_stream : c->stream;
-    EnergyView ev;
-    memset(&ev, 0, sizeof ev);
-    const int newest = c->cur, prev = c->old;
-    if (c->esz == 8) {
-        ev.m = make_view<double>(c, newest, prev, prev);
-    } else {
-        int rc = ensure_scratch(c, (size_t)c->cells * sizeof(double) * 6);
-        if (rc) return rc;
-        double* w = (double*)c->scratch;
-        unsigned g = (unsigned)((c->cells + 255) / 256);
-        for (int l = 0; l < 2; l++)
-            for (int q = 0; q < 3; q++) {
-                int lv = l == 0 ? newest : prev;
-                hipLaunchKernelGGL((k_widen<float>), dim3(g), dim3(256), 0, s, (const float*)c->lvl[lv][q],
-                                   (const lo_t*)c->lvlo[lv][q], w + (size_t)(3 * l + q) * c->cells, c->cells);
-            }
-        HIPCHK(hipGetLastError());
-        Mesh<double>& m = ev.m;
-        memset(&m, 0, sizeof m);
-        m.nx = c->nx; m.ny = c->ny; m.nz = c->nz; m.pz = c->pz; m.plane = c->plane;
-        m.c0 = w; m.c1 = w + c->cells; m.c2 = w + 2 * c->cells;
-        m.n0 = w + 3 * c->cells; m.n1 = w + 4 * c->cells; m.n2 = w + 5 * c->cells;
-        m.ids = c->ids;
+    // about 8 blocks per CU, 4 to ENERGY_XCHUNK planes each
+    const long long per = (c->plane + 255) / 256;
+    long long want = (2048 + per - 1) / per;
+    if (want > (c->nx + 3) / 4) want = (c->nx + 3) / 4;
+    int xc = (int)((c->nx + want - 1) / want);
+    if (xc > ENERGY_XCHUNK) xc = ENERGY_XCHUNK;
+    const long long blocks = per * ((c->nx + xc - 1) / xc);
+    if (blocks > 0x7fffffffLL) return fail(PF_ERR_ARG, "mesh too large for the energy audit");
+    const dim3 grid((unsigned)blocks);
+    if (!c->e_partials) HIPCHK(hipMalloc((void**)&c->e_partials, 2 * sizeof(double) * (size_t)blocks));
+    if (!c->e_out) HIPCHK(hipHostMalloc((void**)&c->e_out, 2 * sizeof(double), hipHostMallocDefault));
+    EnergyArgs ea;
+    ea.mat = (const double*)c->mat64;
+    ea.rho = (const double*)c->rho64;
+    ea.fx = (const double*)c->fx64; ea.fy = (const double*)c->fy64; ea.fz = (const double*)c->fz64;
+    ea.sx = (const double*)c->sx64; ea.sy = (const double*)c->sy64; ea.sz = (const double*)c->sz64;
+    for (int a = 0; a < 3; a++) {
+        ea.f0[a] = c->f0[a];
+        ea.s0[a] = c->s0[a];
     }
-    Mesh<double>& m = ev.m;
-    m.mat = (const double*)c->mat64;
-    m.fx = (const double*)c->fx64; m.fy = (const double*)c->fy64; m.fz = (const double*)c->fz64;
-    m.sx = (const double*)c->sx64; m.sy = (const double*)c->sy64; m.sz = (const double*)c->sz64;
-    m.fx0 = c->f0[0]; m.fy0 = c->f0[1]; m.fz0 = c->f0[2];
-    m.sx0 = c->s0[0]; m.sy0 = c->s0[1]; m.sz0 = c->s0[2];
-    ev.rho = (const double*)c->rho64;
-    ev.dt = c->dt;
-    const long long done = c->step;
-    ev.subst_prev = done > 0 ? 1 : 0;
-    if (done > 0) HIPCHK(hipMemcpy(&ev.w_prev, c->wave + (done - 1), sizeof(double), hipMemcpyDeviceToHost));
-    hipLaunchKernelGGL(k_energy_partial, dim3(c->e_blocks), dim3(256), 0, s, ev, c->e_partials);
-    hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(256), 0, s, (const double*)c->e_partials, c->e_blocks, c->e_out);
+    ea.dt = c->dt;
+    ea.w_prev = c->step > 0 ? c->wave + (c->step - 1) : nullptr;
+    ea.xchunk = xc;
+    ea.per = (unsigned)per;
+    int rc;
+    if (c->precision == PF_FP64) rc = launch_energy<double, false>(c, ea, grid, s);
+    else if (c->precision == PF_FP32) rc = launch_energy<float, false>(c, ea, grid, s);
+    else rc = launch_energy<float, true>(c, ea, grid, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(1024), 0, s, (const double*)c->e_partials, blocks, c->e_out);
     HIPCHK(hipGetLastError());
-    double h[2];
-    HIPCHK(hipMemcpyAsync(h, c->e_out, sizeof h, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    *out = 0.5 * c->dV * (h[0] + h[1]);
+    HIPCHK(hipStreamSynchronize(s));  // the sums land in pinned host memory
+    *out = 0.5 * c->dV * (c->e_out[0] + c->e_out[1]);
     return PF_OK;
 }
 

@@ -95,9 +95,10 @@ struct pf_ctx {
     int every = 0, cap = 0;
     double* ring = nullptr;
     long long* d_frame = nullptr;  // [0] frames recorded; [1], as an int: blocks done in the probe launch
+    // energy audit, allocated by its first call: the two sums (pinned host
+    // memory) and the blocks' partial sums
     double* e_out = nullptr;
     double* e_partials = nullptr;
-    int e_blocks = 0;
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
     pf_batch* batch = nullptr;  // set while a batch owns the stepping
