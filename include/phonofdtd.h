@@ -140,6 +140,11 @@ typedef struct pf_desc {
     int32_t surface;
 } pf_desc;
 
+/* Frees the pinned staging memory that transfers keep between calls (at most
+   8 MiB a device; all but 1 MiB of it also goes with a device's last
+   context). */
+int pf_trim(void);
+
 /* Library / device identification. */
 int pf_abi_version(void);
 const char *pf_last_error(void);

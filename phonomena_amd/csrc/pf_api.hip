@@ -19,6 +19,7 @@
 #include "pf_raster.hpp"
 #include "pf_tiled.hpp"
 #include "pf_block.hpp"
+#include "pf_stage.hpp"
 
 using namespace pf;
 
@@ -189,6 +190,7 @@ extern "C" int pf_create(const pf_desc* d, pf_ctx** out) {
         delete c;
         return rc;
     }
+    stage_users(c->dev, 1);
     *out = c;
     return PF_OK;
 }
@@ -491,8 +493,10 @@ extern "C" int pf_destroy(pf_ctx* c) {
     if (!c) return PF_OK;
     if (c->batch) return fail(PF_ERR_STATE, "context is still a member of a batch");
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    const int dev = c->dev;
     ctx_free(c);
     delete c;
+    stage_users(dev, -1);
     return PF_OK;
 }
 
@@ -893,6 +897,38 @@ static void extents(const pf_ctx* c, int q, int& ex, int& ey, int& ez) {
     ez = c->nz - (q == 2);
 }
 
+// Elements first .. first + count - 1 of component q of level lvl, in the
+// reference's shape, to out on stream s (out may be pinned host memory);
+// wsub: the value for the uz wall line, or null.
+static hipError_t pack(const pf_ctx* c, int lvl, int q, long long first, long long count, double* out,
+                       const double* wsub, hipStream_t s) {
+    int ex, ey, ez;
+    extents(c, q, ex, ey, ez);
+    const dim3 g((unsigned)((count + 255) / 256));
+    if (c->esz == 8)
+        hipLaunchKernelGGL((k_pack<double>), g, dim3(256), 0, s, (const double*)c->lvl[lvl][q], (const lo_t*)nullptr,
+                           c->plane, c->pz, ey, ez, first, count, out, wsub);
+    else
+        hipLaunchKernelGGL((k_pack<float>), g, dim3(256), 0, s, (const float*)c->lvl[lvl][q],
+                           (const lo_t*)c->lvlo[lvl][q], c->plane, c->pz, ey, ez, first, count, out, wsub);
+    return hipGetLastError();
+}
+
+// The same elements from in to the component.
+static hipError_t unpack(pf_ctx* c, int lvl, int q, long long first, long long count, const double* in,
+                         hipStream_t s) {
+    int ex, ey, ez;
+    extents(c, q, ex, ey, ez);
+    const dim3 g((unsigned)((count + 255) / 256));
+    if (c->esz == 8)
+        hipLaunchKernelGGL((k_unpack<double>), g, dim3(256), 0, s, (double*)c->lvl[lvl][q], (lo_t*)nullptr, c->plane,
+                           c->pz, ey, ez, first, count, in);
+    else
+        hipLaunchKernelGGL((k_unpack<float>), g, dim3(256), 0, s, (float*)c->lvl[lvl][q], (lo_t*)c->lvlo[lvl][q],
+                           c->plane, c->pz, ey, ez, first, count, in);
+    return hipGetLastError();
+}
+
 static int ensure_scratch(pf_ctx* c, size_t bytes) {
     if (c->scratch_bytes >= bytes) return PF_OK;
     if (c->scratch) HIPCHK(hipFree(c->scratch));
@@ -940,15 +976,7 @@ extern "C" int pf_snapshot(pf_ctx* c, int32_t slot) {
         int ex, ey, ez;
         extents(c, q, ex, ey, ez);
         const long long n = (long long)ex * ey * ez;
-        const unsigned g = (unsigned)((n + 255) / 256);
-        if (c->esz == 8)
-            hipLaunchKernelGGL((k_pack<double>), dim3(g), dim3(256), 0, c->stream, (const double*)c->lvl[c->cur][q],
-                               (const lo_t*)nullptr, c->plane, c->pz, ex, ey, ez, dev + off, (const double*)nullptr);
-        else
-            hipLaunchKernelGGL((k_pack<float>), dim3(g), dim3(256), 0, c->stream, (const float*)c->lvl[c->cur][q],
-                               (const lo_t*)c->lvlo[c->cur][q], c->plane, c->pz, ex, ey, ez, dev + off,
-                               (const double*)nullptr);
-        HIPCHK(hipGetLastError());
+        HIPCHK(pack(c, c->cur, q, 0, n, dev + off, nullptr, c->stream));
         off += n;
     }
     // the copy waits for the packing only; later steps on the context's
@@ -993,28 +1021,18 @@ extern "C" int pf_get_ids(pf_ctx* c, uint8_t* host, int64_t count) {
     return PF_OK;
 }
 
-// Field `which` into host[0 .. count): packed to FP64 in the reference's
-// shape into the device staging buffer `stage` (count doubles), then copied.
-static int get_field_via(pf_ctx* c, int32_t which, double* host, int64_t count, double* stage) {
-    const int q = which % 3;
-    const int lvl = which < 3 ? c->cur : c->old;
-    int ex, ey, ez;
-    extents(c, q, ex, ey, ez);
-    const long long n = (long long)ex * ey * ez;
-    // the previous level of uz holds the source value on its wall line, as
-    // the reference's u_old does after time_step
-    const double* wsub = (which == PF_UZ_OLD && c->step > 0) ? c->wave + (c->step - 1) : nullptr;
-    unsigned g = (unsigned)((n + 255) / 256);
-    if (c->esz == 8)
-        hipLaunchKernelGGL((k_pack<double>), dim3(g), dim3(256), 0, c->stream, (const double*)c->lvl[lvl][q],
-                           (const lo_t*)nullptr, c->plane, c->pz, ex, ey, ez, stage, wsub);
-    else
-        hipLaunchKernelGGL((k_pack<float>), dim3(g), dim3(256), 0, c->stream, (const float*)c->lvl[lvl][q],
-                           (const lo_t*)c->lvlo[lvl][q], c->plane, c->pz, ex, ey, ez, stage, wsub);
-    HIPCHK(hipGetLastError());
+// The source value that the previous level of uz holds on its wall line, as
+// the reference's u_old does after time_step (null: none).
+static const double* wall_source(const pf_ctx* c, int32_t which) {
+    return which == PF_UZ_OLD && c->step > 0 ? c->wave + (c->step - 1) : nullptr;
+}
+
+// Field `which` into host[0 .. n): packed to FP64 in the reference's shape
+// into the device staging buffer `stage` (n doubles), then copied.
+static int get_field_via(pf_ctx* c, int32_t which, double* host, long long n, double* stage) {
+    HIPCHK(pack(c, which < 3 ? c->cur : c->old, which % 3, 0, n, stage, wall_source(c, which), c->stream));
     HIPCHK(hipMemcpyAsync(host, stage, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    (void)count;
     return PF_OK;
 }
 
@@ -1034,8 +1052,16 @@ extern "C" int pf_get_field(pf_ctx* c, int32_t which, double* host, int64_t coun
     int rc = check_field(c, which, host, count, &n);
     if (rc) return rc;
     if (c->batch) HIPCHK(hipStreamSynchronize(c->batch_stream));
+    // packed chunk by chunk straight into pinned memory
+    const int lvl = which < 3 ? c->cur : c->old, q = which % 3;
+    const double* const w = wall_source(c, which);
+    bool taken = false;
+    rc = stage_out(c->dev, c->stream, host, (size_t)n * sizeof(double), [=](hipStream_t s, char* dst, size_t off, size_t len) {
+        return pack(c, lvl, q, (long long)(off / sizeof(double)), (long long)(len / sizeof(double)), (double*)dst, w, s);
+    }, &taken);
+    if (taken) return rc;
     if ((rc = ensure_scratch(c, (size_t)n * sizeof(double)))) return rc;
-    return get_field_via(c, which, host, count, (double*)c->scratch);
+    return get_field_via(c, which, host, n, (double*)c->scratch);
 }
 
 // ------------------------------------------- allocation-free transfer ----
@@ -1075,7 +1101,7 @@ extern "C" int pf_get_field_noalloc(pf_ctx* c, int32_t which, double* host, int6
     }
     if (!stage) return fail(PF_ERR_STATE, "no staging array on device %d", c->dev);
     if (c->batch) HIPCHK(hipStreamSynchronize(c->batch_stream));
-    return get_field_via(c, which, host, count, stage);
+    return get_field_via(c, which, host, n, stage);
 }
 
 extern "C" int pf_set_field(pf_ctx* c, int32_t which, const double* host, int64_t count) {
@@ -1088,17 +1114,14 @@ extern "C" int pf_set_field(pf_ctx* c, int32_t which, const double* host, int64_
     extents(c, q, ex, ey, ez);
     const long long n = (long long)ex * ey * ez;
     if (count != n) return fail(PF_ERR_ARG, "field %d has %lld elements, got %lld", which, n, (long long)count);
-    int rc = ensure_scratch(c, (size_t)n * sizeof(double));
-    if (rc) return rc;
+    bool taken = false;
+    int rc = stage_in(c->dev, c->stream, host, (size_t)n * sizeof(double), [=](hipStream_t s, const char* src, size_t off, size_t len) {
+        return unpack(c, lvl, q, (long long)(off / sizeof(double)), (long long)(len / sizeof(double)), (const double*)src, s);
+    }, &taken);
+    if (taken) return rc;
+    if ((rc = ensure_scratch(c, (size_t)n * sizeof(double)))) return rc;
     HIPCHK(hipMemcpyAsync(c->scratch, host, (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    unsigned g = (unsigned)((n + 255) / 256);
-    if (c->esz == 8)
-        hipLaunchKernelGGL((k_unpack<double>), dim3(g), dim3(256), 0, c->stream, (double*)c->lvl[lvl][q],
-                           (lo_t*)nullptr, c->plane, c->pz, ex, ey, ez, (const double*)c->scratch);
-    else
-        hipLaunchKernelGGL((k_unpack<float>), dim3(g), dim3(256), 0, c->stream, (float*)c->lvl[lvl][q],
-                           (lo_t*)c->lvlo[lvl][q], c->plane, c->pz, ex, ey, ez, (const double*)c->scratch);
-    HIPCHK(hipGetLastError());
+    HIPCHK(unpack(c, lvl, q, 0, n, (const double*)c->scratch, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return PF_OK;
 }
@@ -1108,19 +1131,22 @@ extern "C" int pf_get_probes(pf_ctx* c, double* host, int64_t cap_frames, int64_
     if (!c || !nframes) return fail(PF_ERR_ARG, "NULL argument");
     *nframes = 0;
     if (c->probe[2] <= 0) return PF_OK;
-    hipStream_t s = c->batch ? c->batch_stream : c->stream;
-    HIPCHK(hipStreamSynchronize(s));
-    long long f = 0;
-    HIPCHK(hipMemcpy(&f, c->d_frame, sizeof f, hipMemcpyDeviceToHost));
+    const long long f = c->step / c->every;  // every recording step since step 0 took a frame
     const long long per = (long long)c->probe[2] * c->probe[5];
     const long long have = f < c->cap ? f : c->cap;
     const long long first = f - have;  // oldest frame still in the ring
     const long long take = have < cap_frames ? have : cap_frames;
     if (take > 0 && !host) return fail(PF_ERR_ARG, "host is NULL");
-    for (long long t = 0; t < take; t++) {
-        long long slot = (first + t) % c->cap;
-        HIPCHK(hipMemcpy(host + t * per, c->ring + slot * per, (size_t)per * sizeof(double), hipMemcpyDeviceToHost));
+    hipStream_t s = c->batch ? c->batch_stream : c->stream;
+    // the frames are two runs of the ring at most
+    for (long long t = 0; t < take;) {
+        const long long slot = (first + t) % c->cap;
+        const long long run = c->cap - slot < take - t ? c->cap - slot : take - t;
+        const int rc = copy_out(c->dev, s, host + t * per, c->ring + slot * per, (size_t)(run * per) * sizeof(double));
+        if (rc) return rc;
+        t += run;
     }
+    if (take <= 0) HIPCHK(hipStreamSynchronize(s));
     *nframes = take;
     return PF_OK;
 }

@@ -733,14 +733,15 @@ static __global__ void k_advance(long long* counter, long long by, long long cap
 }
 
 // ------------------------------------------------------- pack/unpack ----
-// Dense reference-shaped double array <-> padded device component.
+// Dense reference-shaped double array <-> padded device component: elements
+// first .. first + count - 1 of the array, at out[0 ..] / from in[0 ..].
 template <class R>
 __global__ void k_pack(const R* __restrict__ hi, const lo_t* __restrict__ lo, long long plane, int pz,
-                       int ex, int ey, int ez, double* __restrict__ out,
+                       int ey, int ez, long long first, long long count, double* __restrict__ out,
                        const double* __restrict__ wsub) {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    long long n = (long long)ex * ey * ez;
-    if (t >= n) return;
+    const long long o = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (o >= count) return;
+    const long long t = first + o;
     int k = (int)(t % ez);
     long long r = t / ez;
     int j = (int)(r % ey);
@@ -750,21 +751,21 @@ __global__ void k_pack(const R* __restrict__ hi, const lo_t* __restrict__ lo, lo
     double v = (double)h;
     if (lo) v += (double)lo_decode(h, lo[id]);
     if (wsub && i == 0 && k == 0) v = *wsub;  // the source value on the wall line
-    out[t] = v;
+    out[o] = v;
 }
 
 template <class R>
 __global__ void k_unpack(R* __restrict__ hi, lo_t* __restrict__ lo, long long plane, int pz,
-                         int ex, int ey, int ez, const double* __restrict__ in) {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    long long n = (long long)ex * ey * ez;
-    if (t >= n) return;
+                         int ey, int ez, long long first, long long count, const double* __restrict__ in) {
+    const long long o = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (o >= count) return;
+    const long long t = first + o;
     int k = (int)(t % ez);
     long long r = t / ez;
     int j = (int)(r % ey);
     int i = (int)(r / ey);
     long long id = (long long)i * plane + (long long)j * pz + k;
-    double v = in[t];
+    double v = in[o];
     R h = (R)v;
     hi[id] = h;
     if (lo) lo[id] = lo_encode(h, (R)(v - (double)h));

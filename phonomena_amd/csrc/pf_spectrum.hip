@@ -54,6 +54,7 @@
 
 #include "../../include/phonofdtd.h"
 #include "pf_runtime.hpp"
+#include "pf_stage.hpp"
 
 using namespace pf;
 
@@ -452,8 +453,10 @@ int dft_run(const double* in_re, const double* in_im, int pairs, long long batch
     const long long entries = std::max({(1ll << tlg), blue ? n : 0ll, 1ll << lg2});
     hipLaunchKernelGGL(k_fft_tables, dim3((unsigned)((entries + 255) / 256)), dim3(256), 0, nullptr, tables);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpy(base + o_re, in_re, in_bytes, hipMemcpyHostToDevice));
-    if (in_im) HIPCHK(hipMemcpy(base + o_im, in_im, in_bytes, hipMemcpyHostToDevice));
+    int dev = 0, rc;
+    HIPCHK(hipGetDevice(&dev));
+    if ((rc = copy_in(dev, nullptr, base + o_re, in_re, in_bytes))) return rc;
+    if (in_im && (rc = copy_in(dev, nullptr, base + o_im, in_im, in_bytes))) return rc;
     if (window) HIPCHK(hipMemcpy(base + o_win, window, (size_t)n * sizeof(double), hipMemcpyHostToDevice));
     const double* const dre = (const double*)(base + o_re);
     Traces in = {dre, pairs ? dre + 1 : in_im ? (const double*)(base + o_im) : nullptr,
@@ -461,7 +464,6 @@ int dft_run(const double* in_re, const double* in_im, int pairs, long long batch
     double* const ore = (double*)(base + o_ore);
     Spectra out = {ore, out_im ? (double*)(base + o_oim) : ore + 1, nf, out_step, blue ? scale / (double)M : scale};
 
-    int rc;
     if (small) {
         if (blue && (rc = small_launch(lg, 1, in, ch, nullptr, tw, out, bh))) return rc;
         if ((rc = small_launch(lg, batch, in, ch, bh, tw, out, nullptr))) return rc;
@@ -498,8 +500,8 @@ int dft_run(const double* in_re, const double* in_im, int pairs, long long batch
             HIPCHK(hipGetLastError());
         }
     }
-    HIPCHK(hipMemcpy(out_re, base + o_ore, out_bytes, hipMemcpyDeviceToHost));
-    if (out_im) HIPCHK(hipMemcpy(out_im, base + o_oim, out_bytes, hipMemcpyDeviceToHost));
+    if ((rc = copy_out(dev, nullptr, out_re, base + o_ore, out_bytes))) return rc;
+    if (out_im && (rc = copy_out(dev, nullptr, out_im, base + o_oim, out_bytes))) return rc;
     return PF_OK;
 }
 

@@ -103,6 +103,7 @@ def load(path=None):
         "pf_batch_autotune": ([V, I32, P(I32), P(I32), P(I32), P(D)], ctypes.c_int),
         "pf_batch_destroy": ([V], ctypes.c_int),
         "pf_stream_probe": ([I32, I32, I64, I32, P(D), P(D)], ctypes.c_int),
+        "pf_trim": ([], ctypes.c_int),
         "pf_dft": ([V, V, I64, I64, I64, V, D, V, V], ctypes.c_int),
         "pf_dft_complex": ([V, I32, I64, I64, I64, V, D, V], ctypes.c_int),
     }
