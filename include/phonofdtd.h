@@ -267,7 +267,7 @@ int pf_batch_step(pf_batch *b, int64_t nsteps);  /* asynchronous            */
 int pf_batch_sync(pf_batch *b);
 /* Tile shape of the batched sweep: rows (tile_j) x lanes along z (tile_z:
    16x64, 8x64, 32x32, 16x32, 8x32; 0 = default), planes per x chunk
-   (tile_x, 0 = 32), and whether steps are replayed from a HIP graph. */
+   (tile_x, 0 = by the members' work), and whether steps are replayed from a HIP graph. */
 int pf_batch_set_tiles(pf_batch *b, int32_t tile_j, int32_t tile_z, int32_t tile_x, int32_t use_graph);
 /* Autotuner: times every candidate shape over trial_steps real steps (all
    shapes give the same bits, so the members simply advance) and keeps the

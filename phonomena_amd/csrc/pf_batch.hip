@@ -223,14 +223,49 @@ void free_tables(pf_batch* b) {
     b->mem_bytes = b->items_cap = b->nmem_cap = b->fmap_cap = 0;
 }
 
-// Default shapes of a batch (the autotuner refines them).
-void default_shape(const pf_batch* b, int& tj, int& tz, int& tx) {
+// Default rows x lanes of a batch (the autotuner refines them): 16 x 32, 8 x
+// 32 in FP64.  Members are a few times 30 nodes deep, so 62-lane tiles leave
+// lanes idle, and 32 rows make few work items of a small batch.  Measured,
+// microseconds a step at each shape's best chunk, 16 x 32 / 16 x 64 / 8 x 64 /
+// 32 x 32 / 8 x 32: 16 members of 14.2 M nodes FP32C 312 / 315 / 312 / 315 /
+// 335; 10 of 2.8 M 88 / 92 / 95 / 91 / 92; 5 of 1.4 M 64 / 61 / 67 / 62 / 67.
+// From 2^25 nodes on, where every shape keeps the chip full, 16 x 64 (FP32 and
+// FP32C), which reads fewer halo lines: 64 members of 56.6 M nodes FP32 635 us
+// against 651, FP32C 1087 against 1098.  A caller that gives one of the two gets the other as it always was: 64
+// lanes (32 in FP64), 16 rows of 64 or 32 of 32 (8 in FP64).
+void resolve_shape(int precision, long long nodes, int& tj, int& tz) {
+    const bool f64 = precision == PF_FP64;
+    if (tj == 0 && tz == 0) {
+        tj = f64 ? 8 : 16;
+        tz = f64 || nodes < (1ll << 25) ? 32 : 64;
+    }
+    if (tz == 0) tz = f64 ? 32 : 64;
+    if (tj == 0) tj = f64 ? 8 : (tz == 64 ? 16 : 32);
+}
+
+void batch_shape(const pf_batch* b, int& tj, int& tz) {
     tj = b->tile_j;
     tz = b->tile_z;
-    tx = b->tile_x;
-    if (tz == 0) tz = b->precision == PF_FP64 ? 32 : 64;
-    if (tj == 0) tj = b->precision == PF_FP64 ? 8 : (tz == 64 ? 16 : 32);
-    if (tx == 0) tx = 32;
+    long long nodes = 0;
+    for (const pf_ctx* c : b->members) nodes += c->cells;
+    resolve_shape(b->precision, nodes, tj, tz);
+}
+
+// Default planes per chunk: about 1.5 work items per resident block, so that
+// the queues even out uneven members and no CU runs two chunks while another
+// runs none, within 8 (shorter chunks repeat too many warm-up planes) and 32
+// (longer ones gain nothing).  Measured at 8 / 12 / 16 / 24 / 32 / 48 planes,
+// 16 x 32 FP32C: 5 members of 1.4 M nodes 65 / 64 / 70 / 84 / 91 / 108 us a
+// step (the rule: 8), 10 of 2.8 M 89 / 88 / 91 / 93 / 119 / 127 (17), 16 of
+// 14.2 M 330 / 318 / 314 / 312 / 312 / 328 (32).
+int default_xchunk(const pf_batch* b, int tj, int tz) {
+    double planes = 0;  // tile planes of all members
+    for (const pf_ctx* c : b->members) {
+        const TileMap tm = tile_map(c, tj, tz, 1);
+        planes += (double)tm.nkt * tm.njt * c->nx;
+    }
+    const int tx = (int)(planes / (1.5 * b->grid) + 0.5);
+    return tx < 8 ? 8 : tx > 32 ? 32 : tx;
 }
 
 bool shape_built(int tj, int tz) {
@@ -259,8 +294,11 @@ int sweep_grid_s(pf_batch* b, int tj, int tz) {
 
 template <class R, int MODE>
 int build_t(pf_batch* b) {
-    int tj, tz, tx;
-    default_shape(b, tj, tz, tx);
+    int tj, tz;
+    batch_shape(b, tj, tz);
+    int rc = b->sponge == 1 ? sweep_grid_s<R, MODE, true>(b, tj, tz) : sweep_grid_s<R, MODE, false>(b, tj, tz);
+    if (rc) return rc;
+    const int tx = b->tile_x ? b->tile_x : default_xchunk(b, tj, tz);
     const int nmem = (int)b->members.size();
     std::vector<BMember<R>> mem((size_t)nmem);
     std::vector<WorkItem> items;
@@ -360,8 +398,6 @@ int build_t(pf_batch* b) {
         HIPCHK(hipMemcpy(c->d_step, &c->step, sizeof(long long), hipMemcpyHostToDevice));
     }
     b->face_blocks = fblk[(size_t)nmem];
-    int rc = b->sponge == 1 ? sweep_grid_s<R, MODE, true>(b, tj, tz) : sweep_grid_s<R, MODE, false>(b, tj, tz);
-    if (rc) return rc;
     if ((rc = free_graph(b))) return rc;
     b->dirty = false;
     return PF_OK;
@@ -394,8 +430,8 @@ void launch_sweep_s(pf_batch* b, int tj, int tz) {
 // Issue one batched step (three launches) on the batch stream.
 template <class R, int MODE>
 int issue_step_t(pf_batch* b) {
-    int tj, tz, tx;
-    default_shape(b, tj, tz, tx);
+    int tj, tz;
+    batch_shape(b, tj, tz);
     const int nmem = (int)b->members.size();
     if (b->sponge == 1) launch_sweep_s<R, MODE, true>(b, tj, tz);
     else launch_sweep_s<R, MODE, false>(b, tj, tz);
@@ -538,8 +574,7 @@ extern "C" int pf_batch_sync(pf_batch* b) {
 extern "C" int pf_batch_set_tiles(pf_batch* b, int32_t tile_j, int32_t tile_z, int32_t tile_x, int32_t use_graph) {
     if (!b) return fail(PF_ERR_ARG, "batch is NULL");
     int tj = tile_j, tz = tile_z;
-    if (tz == 0) tz = b->precision == PF_FP64 ? 32 : 64;
-    if (tj == 0) tj = b->precision == PF_FP64 ? 8 : (tz == 64 ? 16 : 32);
+    resolve_shape(b->precision, 0, tj, tz);
     if (!shape_built(tj, tz)) return fail(PF_ERR_ARG, "batch tile shape %d rows x %d lanes is not built", tj, tz);
     if (tile_x < 0 || tile_x > XT - 3) return fail(PF_ERR_ARG, "tile_x must be 0..%d", XT - 3);
     HIPCHK(hipStreamSynchronize(b->stream));
