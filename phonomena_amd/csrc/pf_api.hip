@@ -147,11 +147,63 @@ static bool pow2_spacings(const pf_desc* d) {
     return true;
 }
 
+// Whether quotient()'s three operations (pf_formulas.hpp) give RN(a / h) for
+// every dividend a.  With h = B 2^e and a = A 2^f, B and A integers of 53 bits,
+// a quotient near a rounding boundary M (an odd integer of 54 bits, half an
+// ulp its unit) has A 2^w = B M + t, w = 53 or 54, with |t| / 2B its distance
+// in ulp.  The operations' error before the last rounding is below 2^-51 ulp
+// (1.5 ulp of the first quotient times the relative errors of 1 / h and of the
+// remainder), so only |t| <= 8 matters; the dividends of |t| <= 16 are found
+// from M = -t / B mod 2^w and tried.
+static bool quotient_exact(double h) {
+    int e = 0;
+    const uint64_t B = (uint64_t)std::ldexp(std::frexp(h, &e), 53);
+    const double b = (double)B, y = 1.0 / b;
+    const int z = __builtin_ctzll(B);
+    if (z > 4) return true;  // then |t| is 0 or above 16
+    uint64_t inv = B >> z;   // (B / 2^z)^-1 mod 2^64, by Newton's steps
+    for (int k = 0; k < 6; k++) inv *= 2 - (B >> z) * inv;
+    for (int w = 53; w <= 54; w++)
+        for (int t = -16; t <= 16; t++) {
+            if (t == 0 || t % (1 << z)) continue;
+            const uint64_t mod = 1ull << (w - z), lo = 1ull << 53;
+            uint64_t M = ((uint64_t)(int64_t)(-t / (1 << z)) * inv) & (mod - 1);
+            if (M < lo) M += (lo - M + mod - 1) / mod * mod;
+            for (; M < 2 * lo; M += mod) {
+                const uint64_t A = (uint64_t)(((unsigned __int128)B * M + (__int128)t) >> w);
+                if (A < lo / 2 || A >= lo) continue;
+                const double a = (double)A, q = a * y;
+                if (std::fma(std::fma(-b, q, a), y, q) != a / b) return false;
+            }
+        }
+    return true;
+}
+
+// Whether quotient() (pf_formulas.hpp) is exact on this mesh for every
+// displacement in its range: spacings within 2^-60 .. 2^20 that quotient_exact
+// holds for, stiffness entries 0 or within 2^-20 .. 2^100.
+static bool quotients_allowed(const pf_desc* d) {
+    const double* t[6] = {d->fdx, d->fdy, d->fdz, d->sdx, d->sdy, d->sdz};
+    const int n[6] = {d->nx - 1, d->ny - 1, d->nz - 1, d->nx - 2, d->ny - 2, d->nz - 2};
+    for (int a = 0; a < 6; a++)
+        for (int i = 0; i < n[a]; i++) {
+            const double h = t[a][i];
+            if (i > 0 && h == t[a][i - 1]) continue;
+            if (!(h >= 0x1p-60 && h <= 0x1p20) || !quotient_exact(h)) return false;
+        }
+    for (int r = 0; r < d->n_materials; r++)
+        for (int q = 0; q < 12; q++) {
+            const double v = std::fabs(d->materials[r * 13 + q]);
+            if (!(v == 0 || (v >= 0x1p-20 && v <= 0x1p100))) return false;
+        }
+    return true;
+}
+
 template <class R>
 static int create_tables(pf_ctx* c, const pf_desc* d) {
     const bool exact = d->precision == PF_FP64;
     int rc;
-    if (c->recip) {
+    if (exact) {
         if ((rc = upload_table(&c->rfx, spacing_table<double>(d->fdx, d->nx - 1, true)))) return rc;
         if ((rc = upload_table(&c->rfy, spacing_table<double>(d->fdy, d->ny - 1, true)))) return rc;
         if ((rc = upload_table(&c->rfz, spacing_table<double>(d->fdz, d->nz - 1, true)))) return rc;
@@ -363,6 +415,7 @@ int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
     // the FP64 one-step tiled sweep and block steps on power-of-two spacings
     // multiply by exact reciprocals (MODE_FP64P)
     c->recip = d->precision == PF_FP64 && c->kernel == PF_KERNEL_TILED && pow2_spacings(d);
+    c->quot = d->precision == PF_FP64 && c->kernel == PF_KERNEL_TILED && !c->recip && quotients_allowed(d);
     if (d->kernel == PF_KERNEL_AUTO && c->kernel == PF_KERNEL_TILED && c->shape_open && c->tile_x == 0) block_plan(c);
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
 
@@ -523,6 +576,12 @@ Mesh<R> pf::make_view(const pf_ctx* c, int cur, int old, int nxt) {
     m.sx0 = (R)(exact ? c->s0[0] : 1.0 / c->s0[0]);
     m.sy0 = (R)(exact ? c->s0[1] : 1.0 / c->s0[1]);
     m.sz0 = (R)(exact ? c->s0[2] : 1.0 / c->s0[2]);
+    if (exact) {
+        m.rfx = (const R*)c->rfx; m.rfy = (const R*)c->rfy; m.rfz = (const R*)c->rfz;
+        m.rsx = (const R*)c->rsx; m.rsy = (const R*)c->rsy; m.rsz = (const R*)c->rsz;
+        m.rfx0 = (R)(1.0 / c->f0[0]); m.rfy0 = (R)(1.0 / c->f0[1]); m.rfz0 = (R)(1.0 / c->f0[2]);
+        m.rsx0 = (R)(1.0 / c->s0[0]); m.rsy0 = (R)(1.0 / c->s0[1]); m.rsz0 = (R)(1.0 / c->s0[2]);
+    }
     m.dpx = (const R*)c->dpx; m.dpy = (const R*)c->dpy; m.dpz = (const R*)c->dpz;
     for (int e = 0; e < 12; e++) {
         m.mur[e] = (R)c->mur[e];
@@ -543,7 +602,7 @@ template Mesh<double> pf::make_view<double>(const pf_ctx*, int, int, int);
 // Launch the sweep of one step of mesh view m on stream s.
 template <class R, int MODE>
 static int launch_sweep_t(const pf_ctx* c, const Mesh<R>& m, hipStream_t s) {
-    if constexpr (MODE == MODE_FP64P) {  // built for the one-step tiled sweep only
+    if constexpr (MODE == MODE_FP64P || MODE == MODE_FP64Q) {  // built for the one-step tiled sweep only
         if (c->kernel != PF_KERNEL_TILED) return fail(PF_ERR_STATE, "reciprocal spacings need the tiled sweep");
         return launch_tiled<R, MODE>(c, m, s);
     } else {
@@ -614,10 +673,10 @@ template <class R, int MODE>
 static Mesh<R> sweep_view(const pf_ctx* c, int cur, int old, int nxt) {
     Mesh<R> m = make_view<R>(c, cur, old, nxt);
     if constexpr (MODE == MODE_FP64P) {
-        m.fx = (const R*)c->rfx; m.fy = (const R*)c->rfy; m.fz = (const R*)c->rfz;
-        m.sx = (const R*)c->rsx; m.sy = (const R*)c->rsy; m.sz = (const R*)c->rsz;
-        m.fx0 = (R)(1.0 / c->f0[0]); m.fy0 = (R)(1.0 / c->f0[1]); m.fz0 = (R)(1.0 / c->f0[2]);
-        m.sx0 = (R)(1.0 / c->s0[0]); m.sy0 = (R)(1.0 / c->s0[1]); m.sz0 = (R)(1.0 / c->s0[2]);
+        m.fx = m.rfx; m.fy = m.rfy; m.fz = m.rfz;
+        m.sx = m.rsx; m.sy = m.rsy; m.sz = m.rsz;
+        m.fx0 = m.rfx0; m.fy0 = m.rfy0; m.fz0 = m.rfz0;
+        m.sx0 = m.rsx0; m.sy0 = m.rsy0; m.sz0 = m.rsz0;
     }
     return m;
 }
@@ -632,8 +691,8 @@ static int step_once_t(pf_ctx* c, hipStream_t s, const long long* base, long lon
     if (ev) HIPCHK(hipEventRecord(ev[0], s));
     if ((rc = launch_sweep_t<R, MODE>(c, m, s))) return rc;
     if (ev) HIPCHK(hipEventRecord(ev[1], s));
-    // the faces read no spacings: the FP64 face kernels serve MODE_FP64P
-    if ((rc = launch_faces_probe_t<R, MODE == MODE_FP64P ? MODE_FP64 : MODE>(c, m, s))) return rc;
+    // the faces read no spacings: the FP64 face kernels serve all FP64 modes
+    if ((rc = launch_faces_probe_t<R, MODE == MODE_FP64P || MODE == MODE_FP64Q ? MODE_FP64 : MODE>(c, m, s))) return rc;
     const int t = c->cur;
     c->cur = c->old;
     c->old = t;
@@ -655,7 +714,7 @@ template <class R, int MODE>
 static int tune_shape_t(pf_ctx* c) {
     static const int f32[][2] = {{16, 64}, {8, 64}, {32, 32}, {16, 32}, {8, 32}};
     static const int f64[][2] = {{8, 32}, {16, 32}, {8, 64}};
-    const bool d64 = MODE == MODE_FP64 || MODE == MODE_FP64P;
+    const bool d64 = sizeof(R) == 8;
     const int (*cand)[2] = d64 ? f64 : f32;
     const int nc = d64 ? 3 : 5;
     if (c->wave_len < 1) return PF_OK;  // the sweep would return at once
@@ -708,7 +767,10 @@ static int tune_shape_t(pf_ctx* c) {
 
 static int tune_shape(pf_ctx* c) {
     switch (c->precision) {
-        case PF_FP64: return c->recip ? tune_shape_t<double, MODE_FP64P>(c) : tune_shape_t<double, MODE_FP64>(c);
+        case PF_FP64:
+            return c->recip  ? tune_shape_t<double, MODE_FP64P>(c)
+                   : c->quot ? tune_shape_t<double, MODE_FP64Q>(c)
+                             : tune_shape_t<double, MODE_FP64>(c);
         case PF_FP32: return tune_shape_t<float, MODE_FP32>(c);
         default: return tune_shape_t<float, MODE_FP32C>(c);
     }
@@ -780,8 +842,9 @@ int pf::step_pair(pf_ctx* c, hipStream_t s, const long long* base, long long off
 int pf::step_once(pf_ctx* c, hipStream_t s, const long long* base, long long off, hipEvent_t* ev) {
     switch (c->precision) {
         case PF_FP64:
-            return c->recip ? step_once_t<double, MODE_FP64P>(c, s, base, off, ev)
-                            : step_once_t<double, MODE_FP64>(c, s, base, off, ev);
+            return c->recip  ? step_once_t<double, MODE_FP64P>(c, s, base, off, ev)
+                   : c->quot ? step_once_t<double, MODE_FP64Q>(c, s, base, off, ev)
+                             : step_once_t<double, MODE_FP64>(c, s, base, off, ev);
         case PF_FP32: return step_once_t<float, MODE_FP32>(c, s, base, off, ev);
         default: return step_once_t<float, MODE_FP32C>(c, s, base, off, ev);
     }
@@ -832,6 +895,9 @@ static int step_block_t(pf_ctx* c, hipStream_t s, long long off, int r, hipEvent
 static int step_block(pf_ctx* c, hipStream_t s, long long off, int r, hipEvent_t* ev) {
     switch (c->precision) {
         case PF_FP64:
+            // (quotients from reciprocals are no gain here: the chain of a step
+            // is latency, and they cost a block registers; 58 x 39 x 13 nodes 9.7
+            // us a step against 8.7)
             return c->recip ? step_block_t<double, MODE_FP64P>(c, s, off, r, ev)
                             : step_block_t<double, MODE_FP64>(c, s, off, r, ev);
         case PF_FP32: return step_block_t<float, MODE_FP32>(c, s, off, r, ev);

@@ -14,6 +14,10 @@
 //    same real number (subnormal and overflowing results included), so this
 //    is bit-identical to flavour 1, for the price of a multiply instead of a
 //    correctly rounded division (about ten instructions in FP64).
+//  * 3 (FP64 parity mode, where values allow it): the correctly rounded
+//    quotient a / h from the spacing's reciprocal, see quotient() below; the
+//    same bits as flavour 1 again (a zero may differ in sign, which no value
+//    of the scheme depends on).
 //  * 0 (FP32 modes): divisions replaced by products with inverse spacings,
 //    explicit fused multiply-adds.
 //
@@ -33,26 +37,85 @@ enum : int { M_C00 = 0, M_C01, M_C02, M_C10, M_C11, M_C12, M_C20, M_C21, M_C22,
 
 // MODE_FP64P: MODE_FP64 on a mesh whose spacings are all powers of two
 // (flavour 2 above); the host picks it, with reciprocal spacing tables.
-enum : int { MODE_FP64 = 0, MODE_FP32 = 1, MODE_FP32C = 2, MODE_FP64P = 3 };
+// MODE_FP64Q: MODE_FP64 with flavour 3 where a block's values allow it and
+// flavour 1 elsewhere; the host picks it when the spacings and stiffnesses do.
+enum : int { MODE_FP64 = 0, MODE_FP32 = 1, MODE_FP32C = 2, MODE_FP64P = 3, MODE_FP64Q = 4 };
 
 // The formula flavour of a mode.
-constexpr int exact_of(int mode) { return mode == MODE_FP64 ? 1 : (mode == MODE_FP64P ? 2 : 0); }
+constexpr int exact_of(int mode) {
+    return mode == MODE_FP64 ? 1 : (mode == MODE_FP64P ? 2 : (mode == MODE_FP64Q ? 3 : 0));
+}
 
 PF_DEV float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 PF_DEV double mad(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// a / h in flavour 1; a * h (h holding 1/h) in flavour 2.
+// A spacing with its reciprocal y = RN(1 / h) (MODE_FP64Q).
+template <class R> struct Div { R h, y; };
+// What a mode's kernels hold for a spacing.
+template <class R, int MODE> struct SpacingOf { typedef R type; };
+template <> struct SpacingOf<double, MODE_FP64Q> { typedef Div<double> type; };
+template <class R, int MODE> using Spacing = typename SpacingOf<R, MODE>::type;
+template <class H, class R> PF_DEV H spacing(R h, R y) {
+    if constexpr (sizeof(H) == sizeof(R)) return h;
+    else return H{h, y};
+}
+
+// RN(a / h) in three operations (Markstein: a quotient from y = RN(1 / h),
+// corrected by its remainder).  q = RN(a y) is within 1.5 ulp of a / h, so the
+// corrected sum differs from a / h by less than 2^-51 ulp before it is
+// rounded, and RN of it is RN(a / h) unless a / h is that near a rounding
+// boundary.  For a given h only a few dividends come so near; the host tries
+// the three operations on all of them (quotient_exact, pf_api.hip) and leaves
+// a mesh with a spacing that fails to the divisions (none was found among
+// 2 x 10^6 random spacings).  This holds while nothing on the way underflows
+// or overflows, which follows from the displacements alone (in_range): with
+// every spacing at most 2^H and every stiffness entry 0 or at least 2^-C,
+// displacements that are 0 or at least 2^-L are multiples of 2^-(L+52),
+// and so are their differences; quotients of those (times a stiffness) are 0
+// or at least 2^-(L+52+C+H) and their sums multiples of 2^-(L+104+C+H), a
+// shear stress, a stiffness times such a sum, of 2^-(L+156+C+H); so the stress
+// differences that the update divides are 0 or at least that, their quotients
+// are normal and their remainders, multiples of 2^-106 times the dividend,
+// exact up to L = 812 - C - 2 H: QUOT_L = 752 for H = C = 20.  Upwards,
+// displacements below 2^400, entries below 2^100 and spacings above 2^-60 keep
+// everything below 2^630.  (A bound per mesh, as a kernel argument, measured 6 %
+// slower than this constant.)
+// The compiler's division takes about 14 issue slots (it scales, takes a
+// quarter-rate reciprocal and fixes special cases up).  A step of the tiled
+// sweep with quotients, with divisions: 205 x 193 x 101 nodes 101 us, 118; with
+// an absorbing layer 121, 129; 257 x 257 x 129 with one 235, 250; 129 x 129 x
+// 65 with one 46, 54.  Noting the range costs 8 of the 101; a second
+// correction, which needs no check of the spacings, 10.
+PF_DEV double quotient(double a, Div<double> d) {
+    const double q = a * d.y;
+    return __builtin_fma(__builtin_fma(-d.h, q, a), d.y, q);
+}
+// Whether a displacement is 0 or within 2^-QUOT_L .. 2^400.
+constexpr int QUOT_L = 752;
+PF_DEV bool in_range(double v) {
+    constexpr unsigned lo = (1023u - QUOT_L) << 20, hi = (1023u + 400u) << 20;
+    const unsigned e = (unsigned)(__double_as_longlong(v) >> 32) & 0x7fffffffu;
+    return e - lo < hi - lo || v == 0.0;
+}
+PF_DEV bool in_range(float) { return true; }
+
+// a / h in flavours 1 and 3; a * h (h holding 1/h) in flavour 2.
 template <int EXACT, class R>
 PF_DEV R over(R a, R h) {
     if constexpr (EXACT == 2) return a * h;
     else return a / h;
 }
+template <int EXACT>
+PF_DEV double over(double a, Div<double> d) {
+    if constexpr (EXACT == 3) return quotient(a, d);
+    else return a / d.h;
+}
 
 // ---- normal stresses T1..T3 -------------------------------------------------
 // Interior (base_solver.py:329-351): row a of C times the three normal
 // differences, each divided by its staggered spacing.
-template <int EXACT, class R>
-PF_DEV void normal3(const R* c, R dux, R duy, R duz, R hx, R hy, R hz, R& t1, R& t2, R& t3) {
+template <int EXACT, class R, class H>
+PF_DEV void normal3(const R* c, R dux, R duy, R duz, H hx, H hy, H hz, R& t1, R& t2, R& t3) {
     if constexpr (EXACT) {
         t1 = over<EXACT>(c[M_C00] * dux, hx) + over<EXACT>(c[M_C01] * duy, hy) + over<EXACT>(c[M_C02] * duz, hz);
         t2 = over<EXACT>(c[M_C10] * dux, hx) + over<EXACT>(c[M_C11] * duy, hy) + over<EXACT>(c[M_C12] * duz, hz);
@@ -86,8 +149,8 @@ PF_DEV void normal3_surface(const R* c, R dux, R duy, R uz0, R hx0, R hy0, R hz0
 // c * (a / h1 + b / h2); the caller passes the spacings in the order the
 // reference divides by them (interior: base_solver.py:353-372, surface with
 // its swapped spacings: :420-433).
-template <int EXACT, class R>
-PF_DEV R shear(R c, R a, R h1, R b, R h2) {
+template <int EXACT, class R, class H>
+PF_DEV R shear(R c, R a, H h1, R b, H h2) {
     if constexpr (EXACT) {
         return c * (over<EXACT>(a, h1) + over<EXACT>(b, h2));
     } else {
@@ -97,8 +160,8 @@ PF_DEV R shear(R c, R a, R h1, R b, R h2) {
 
 // ---- displacement divergence ------------------------------------------------
 // (d1 / g1 + d2 / g2) + d3 / g3  (base_solver.py:444-446 and analogues)
-template <int EXACT, class R>
-PF_DEV R div3(R d1, R g1, R d2, R g2, R d3, R g3) {
+template <int EXACT, class R, class H>
+PF_DEV R div3(R d1, H g1, R d2, H g2, R d3, H g3) {
     if constexpr (EXACT) {
         return over<EXACT>(d1, g1) + over<EXACT>(d2, g2) + over<EXACT>(d3, g3);
     } else {

@@ -68,6 +68,14 @@ struct Mesh {
     const R* __restrict__ sy;
     const R* __restrict__ sz;
     R fx0, fy0, fz0, sx0, sy0, sz0;
+    // FP64: reciprocals of the spacings (the same tables, MODE_FP64Q)
+    const R* __restrict__ rfx;
+    const R* __restrict__ rfy;
+    const R* __restrict__ rfz;
+    const R* __restrict__ rsx;
+    const R* __restrict__ rsy;
+    const R* __restrict__ rsz;
+    R rfx0, rfy0, rfz0, rsx0, rsy0, rsz0;
     const R* __restrict__ dpx;  // sponge terms per axis (null: none)
     const R* __restrict__ dpy;
     const R* __restrict__ dpz;

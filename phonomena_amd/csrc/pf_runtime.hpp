@@ -77,10 +77,11 @@ struct pf_ctx {
     void *mat = nullptr, *fx = nullptr, *fy = nullptr, *fz = nullptr, *sx = nullptr, *sy = nullptr,
          *sz = nullptr;
     void *dpx = nullptr, *dpy = nullptr, *dpz = nullptr;
-    // FP64 with every spacing a power of two: the reciprocal tables of the
-    // one-step tiled sweep's products (MODE_FP64P); fx.. keep the spacings
-    // for the other kernels (batch, energy).
-    bool recip = false;
+    // FP64: the reciprocals of the spacing tables, which fx.. keep.  recip:
+    // every spacing is a power of two, so the tiled sweep and block steps
+    // multiply by them (MODE_FP64P); quot: otherwise they take exact quotients
+    // from them (MODE_FP64Q).
+    bool recip = false, quot = false;
     void *rfx = nullptr, *rfy = nullptr, *rfz = nullptr, *rsx = nullptr, *rsy = nullptr, *rsz = nullptr;
     void *mat64 = nullptr, *rho64 = nullptr, *fx64 = nullptr, *fy64 = nullptr, *fz64 = nullptr,
          *sx64 = nullptr, *sy64 = nullptr, *sz64 = nullptr;

@@ -215,12 +215,14 @@ PF_DEV Old<R> load_old(const Bufs& bf, int i, unsigned plane, unsigned boff, uns
 
 // Per-plane x data staged in LDS: hs = staggered spacing (sx[p-1], 1 off
 // its range), hf = full spacing (fx[p], 1 off its range), dp = sponge term.
-template <class R>
+template <class R, class H = R>
 struct XPlane {
-    R hs, hf, dp, pad;
+    H hs, hf;
+    R dp, pad;
 };
 
 template <class R> PF_DEV R sel(bool c, R a, R b) { return c ? a : b; }
+template <class R> PF_DEV Div<R> sel(bool c, Div<R> a, Div<R> b) { return {c ? a.h : b.h, c ? a.y : b.y}; }
 
 // Own-cell store through the array's buffer descriptor, then, for the top
 // cell of the column (k = Lz - 1), the z = max Mur face cell above it:
@@ -240,7 +242,7 @@ PF_DEV void put_tile(const Mesh<R>& m, const Bufs& bf, unsigned boff, unsigned l
 
 // Shared memory of one block.  Material rows are addressed by byte offset
 // (id * row bytes), which is what the id registers and sid carry.
-template <class R, int TJ, int KZ>
+template <class R, int TJ, int KZ, class H = R>
 struct TiledLds {
     R su[2][3][TJ][KZ];   // u planes, by plane parity
     R sn2[2][TJ][KZ];     // T2 of a plane, by plane parity
@@ -248,7 +250,9 @@ struct TiledLds {
     R ss6[TJ][KZ];        // T6 of the current plane
     uint16_t sid[2][TJ][KZ];
     R smat[PF_TILED_MAX_MATERIALS * MAT_STRIDE];
-    XPlane<R> sxp[XT];    // planes ib-1 .. ie+1
+    XPlane<R, H> sxp[XT]; // planes ib-1 .. ie+1
+    // MODE_FP64Q: whether a wave holds a displacement out of range, by plane & 3
+    uint8_t out[4][TJ * KZ / 64];
 };
 
 template <class R> PF_DEV const R* mrow(const R* smat, int off) {
@@ -281,9 +285,14 @@ PF_DEV double above0(double v) {
 // left out (same bits); the x conditions left in a FYZ block are uniform
 // over the block (per plane).
 template <class R, int MODE, bool SPONGE, int TJ, int KZ, bool FYZ, bool FX>
-PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int row, int k, int j, int ib, int ie,
-                        R w) {
+PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ, Spacing<R, MODE>>& L, int kl, int row, int k, int j,
+                        int ib, int ie, R w) {
     constexpr int EXACT = exact_of(MODE);
+    constexpr bool QUOT = MODE == MODE_FP64Q;
+    typedef Spacing<R, MODE> H;
+    const H one = spacing<H>(R(1), R(1));
+    const H sx0 = spacing<H>(m.sx0, m.rsx0), sy0 = spacing<H>(m.sy0, m.rsy0), sz0 = spacing<H>(m.sz0, m.rsz0);
+    const H fx0 = spacing<H>(m.fx0, m.rfx0), fy0 = spacing<H>(m.fy0, m.rfy0), fz0 = spacing<H>(m.fz0, m.rfz0);
     constexpr bool COMP = MODE == MODE_FP32C;
     constexpr int RB = MAT_STRIDE * (int)sizeof(R);  // bytes per material row
     const int rp = row + 1 < TJ ? row + 1 : TJ - 1;
@@ -304,24 +313,41 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
     const bool kn = FYZ || (k >= 1 && k <= m.nz - 2);
     const bool kf = FYZ || (k >= 0 && k <= m.nz - 2);
     const bool writer = valid && kl >= 1 && kl <= KZ - 2 && row >= 1 && row <= TJ - 2;
-    const R hsy = jn ? m.sy[j - 1] : R(1);
-    const R hfy = jf ? m.fy[j] : R(1);
-    const R hsz = kn ? m.sz[k - 1] : R(1);
-    const R hfz = kf ? m.fz[k] : R(1);
-    const R hy_n = sel(ks, hsy, m.sy0);        // normal stresses, ux update: y
-    const R hz_n = sel(ks, hsz, m.sz0);        // normal stresses, ux/uy update: z
-    const R s4_h1 = sel(ks, hfz, m.fy0), s4_h2 = sel(ks, hfy, m.fz0);
-    const R s5_h1 = sel(ks, hfz, m.fx0);
-    const R s6_h1 = sel(ks, hfy, m.fx0);
-    const R uy_g2 = sel(ks, hfy, m.fy0);
+    auto table = [](const R* h, const R* y, int i) { return spacing<H>(h[i], QUOT ? y[i] : R(0)); };
+    const H hsy = jn ? table(m.sy, m.rsy, j - 1) : one;
+    const H hfy = jf ? table(m.fy, m.rfy, j) : one;
+    const H hsz = kn ? table(m.sz, m.rsz, k - 1) : one;
+    const H hfz = kf ? table(m.fz, m.rfz, k) : one;
+    const H hy_n = sel(ks, hsy, sy0);          // normal stresses, ux update: y
+    const H hz_n = sel(ks, hsz, sz0);          // normal stresses, ux/uy update: z
+    const H s4_h1 = sel(ks, hfz, fy0), s4_h2 = sel(ks, hfy, fz0);
+    const H s5_h1 = sel(ks, hfz, fx0);
+    const H s6_h1 = sel(ks, hfy, fx0);
+    const H uy_g2 = sel(ks, hfy, fy0);
     // u_z's T3 term at k = 0: the reference's unscaled T3[..,1], or (surf)
     // the difference divided by fdz, as in the interior
-    const R uz_g3 = sel(ks || m.surf, hfz, R(1));
+    const H uz_g3 = sel(ks || m.surf, hfz, one);
     R dpyz = R(0), dpz_k = R(0);
     if constexpr (SPONGE) {
         dpyz = m.dpy[j < 0 ? 0 : (j < m.ny ? j : m.ny - 1)];
         dpz_k = m.dpz[k < 0 ? 0 : (k < m.nz ? k : m.nz - 1)];
     }
+    // MODE_FP64Q: a wave notes whether a plane's displacements are out of
+    // quotient()'s range; a block divides where any of its waves' are
+    const int wave = (row * KZ + kl) / 64;
+    auto note = [&](int p, const Col<R>& c) {
+        if constexpr (QUOT) {
+            const bool out = __any(!(in_range(c.x) && in_range(c.y) && in_range(c.z)));
+            if ((threadIdx.x & 63) == 0) L.out[p & 3][wave] = out;
+        }
+    };
+    auto noted = [&](int p) {
+        unsigned v = 0;
+        const unsigned* f = (const unsigned*)L.out[p & 3];
+#pragma unroll
+        for (int g = 0; g < TJ * KZ / 256; g++) v |= f[g];
+        return v;
+    };
     const unsigned col = valid ? (unsigned)(j * m.pz + k) : 0u;
     const unsigned boff = col * (unsigned)sizeof(R);
     const unsigned loff = col * (unsigned)sizeof(lo_t);
@@ -345,6 +371,7 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
     Col<R> c0 = settle(load_raw<R>(bf, ib >= 1 ? ib - 1 : 0, plane, boff, col), valid && ib >= 1,
                        !FYZ && ib - 1 == 0 && k == 0, w);
     c0.id *= RB;
+    note(ib - 1, c0);
     // issue order ra, rb, ob (kept by the scheduling barriers) matches the
     // steady state, so the loop needs no wait for more than it uses
     Raw<R> ra = load_raw<R>(bf, ib, plane, boff, col);
@@ -361,62 +388,69 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
 
     R n1_0 = 0, n2_0 = 0, n3_0 = 0;  // N at plane i
     R s5_m = 0, s6_m = 0;            // T5, T6 at plane i-1
+    unsigned far_m = 0;              // planes i-1 and i were out of range
     const R* smat = L.smat;
 
-    // One plane i: H is the LDS parity of plane i+1, rin holds the raw
+    // One plane i: P is the LDS parity of plane i+1, rin holds the raw
     // column of plane i+1 and receives plane i+3, oin holds the node values
     // of plane i and receives plane i+2.
-    auto plane_step = [&](int i, auto Hc, Raw<R>& rin, Old<R>& oin) {
-        constexpr int H = decltype(Hc)::value;
+    auto plane_step = [&](int i, auto Pc, Raw<R>& rin, Old<R>& oin) {
+        constexpr int P = decltype(Pc)::value;
         const int ip = i + 1;
         Col<R> c1 = settle(rin, valid && (FX || ip < m.nx), !FYZ && ip == 0 && k == 0, w);
         c1.id *= RB;
-        L.su[H][0][row][kl] = c1.x;
-        L.su[H][1][row][kl] = c1.y;
-        L.su[H][2][row][kl] = c1.z;
-        L.sid[H][row][kl] = (uint16_t)c1.id;
+        note(ip, c1);
+        L.su[P][0][row][kl] = c1.x;
+        L.su[P][1][row][kl] = c1.y;
+        L.su[P][2][row][kl] = c1.z;
+        L.sid[P][row][kl] = (uint16_t)c1.id;
         __syncthreads();
         // issued after the barrier, so the registers of rin are free again
         rin = load_raw<R>(bf, ip + 2 <= pmax ? ip + 2 : pmax, plane, boff, col);
 
-        const XPlane<R> xq0 = L.sxp[i - ib + 1];  // x data of plane i
-        const XPlane<R> xq1 = L.sxp[ip - ib + 1];
-        const R uy1_jm = L.su[H][1][rm][kl];
+        const XPlane<R, H> xq0 = L.sxp[i - ib + 1];  // x data of plane i
+        const XPlane<R, H> xq1 = L.sxp[ip - ib + 1];
+        const R uy1_jm = L.su[P][1][rm][kl];
         const R uz1_km = below0(c1.z);
         const R uy0_kp = above0(c0.y);
         const R ux0_kp = above0(c0.x);
-        const R uz0_jp = L.su[1 - H][2][rp][kl];
-        const R ux0_jp = L.su[1 - H][0][rp][kl];
-        const int id_jp = L.sid[1 - H][rp][kl];   // (i, j+1, k)
-        const int id1_jp = L.sid[H][rp][kl];      // (i+1, j+1, k)
+        const R uz0_jp = L.su[1 - P][2][rp][kl];
+        const R ux0_jp = L.su[1 - P][0][rp][kl];
+        const int id_jp = L.sid[1 - P][rp][kl];   // (i, j+1, k)
+        const int id1_jp = L.sid[P][rp][kl];      // (i+1, j+1, k)
         const int id_kp = dpp_above0(c0.id);      // (i, j, k+1)
         const int id_jkp = dpp_above0(id_jp);     // (i, j+1, k+1)
         const int id1_kp = dpp_above0(c1.id);     // (i+1, j, k+1)
 
-        // normal stresses at plane ip (base_solver.py:329-351, 408-418)
-        R n1_1, n2_1, n3_1;
-        {
-            normal3<EXACT>(mrow(smat, c1.id), c1.x - c0.x, c1.y - uy1_jm, c1.z - sel(ks, uz1_km, R(0)),
-                           sel(ks, xq1.hs, m.sx0), hy_n, hz_n, n1_1, n2_1, n3_1);
-            if constexpr (!FULL) {
-                const bool nv = ip >= 1 && ip <= m.nx - 2 && jn && kf;
-                n1_1 = sel(nv, n1_1, R(0));
-                n2_1 = sel(nv, n2_1, R(0));
-                n3_1 = sel(nv && ks, n3_1, R(0));
-            }
-        }
-        // shear stresses at plane i (base_solver.py:353-372, 420-433)
-        const R fxi = sel(ks, xq0.hf, m.fz0);
-        R s4 = shear<EXACT>(mget(smat, ks ? id_jkp : id_jp, M_C33), uy0_kp - c0.y, s4_h1, uz0_jp - c0.z, s4_h2);
-        R s5 = shear<EXACT>(mget(smat, ks ? id1_kp : c1.id, M_C44), ux0_kp - c0.x, s5_h1, c1.z - c0.z, fxi);
-        R s6 = shear<EXACT>(mget(smat, id1_jp, M_C55), ux0_jp - c0.x, s6_h1, c1.y - c0.y, fxi);
+        // the stresses read planes i and ip, the update planes i-1 too
+        unsigned far = 0;  // uniform: a plane is out of quotient()'s range
+        if constexpr (QUOT) far = uni(noted(i) | noted(ip));
+        // normal stresses at plane ip (base_solver.py:329-351, 408-418), shear
+        // stresses at plane i (:353-372, 420-433)
+        R n1_1, n2_1, n3_1, s4, s5, s6;
+        auto stresses = [&](auto Ec) {
+            constexpr int E = decltype(Ec)::value;
+            normal3<E>(mrow(smat, c1.id), c1.x - c0.x, c1.y - uy1_jm, c1.z - sel(ks, uz1_km, R(0)),
+                       sel(ks, xq1.hs, sx0), hy_n, hz_n, n1_1, n2_1, n3_1);
+            const H fxi = sel(ks, xq0.hf, fz0);
+            s4 = shear<E>(mget(smat, ks ? id_jkp : id_jp, M_C33), uy0_kp - c0.y, s4_h1, uz0_jp - c0.z, s4_h2);
+            s5 = shear<E>(mget(smat, ks ? id1_kp : c1.id, M_C44), ux0_kp - c0.x, s5_h1, c1.z - c0.z, fxi);
+            s6 = shear<E>(mget(smat, id1_jp, M_C55), ux0_jp - c0.x, s6_h1, c1.y - c0.y, fxi);
+        };
+        if (QUOT && far) stresses(std::integral_constant<int, 1>());
+        else stresses(std::integral_constant<int, EXACT>());
         if constexpr (!FULL) {
+            const bool nv = ip >= 1 && ip <= m.nx - 2 && jn && kf;
+            n1_1 = sel(nv, n1_1, R(0));
+            n2_1 = sel(nv, n2_1, R(0));
+            n3_1 = sel(nv && ks, n3_1, R(0));
+
             const bool ii = i >= 0 && i <= m.nx - 2;
             s4 = sel(ii && i >= 1 && jf && kf, s4, R(0));
             s5 = sel(ii && jn && kf, s5, R(0));
             s6 = sel(ii && jf && kf, s6, R(0));
         }
-        L.sn2[H][row][kl] = n2_1;
+        L.sn2[P][row][kl] = n2_1;
         L.ss4[row][kl] = s4;
         L.ss6[row][kl] = s6;
         __syncthreads();
@@ -425,11 +459,20 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
         const R s4_km = below0(s4);
         const R s5_km = below0(s5);
         if (i >= ib && i < ie) {
-            const R n2_0_jp = L.sn2[1 - H][rp][kl];
+            const R n2_0_jp = L.sn2[1 - P][rp][kl];
             const R s4_jm = L.ss4[rm][kl];
             const R s6_jm = L.ss6[rm][kl];
             const R s = SPONGE ? (xq0.dp + dpyz) + dpz_k : R(0);
-            const R gx = sel(ks, xq0.hs, m.sx0);
+            const H gx = sel(ks, xq0.hs, sx0);
+            R dvx, dvy, dvz;  // base_solver.py:441-463, 495-517
+            auto divergence = [&](auto Ec) {
+                constexpr int E = decltype(Ec)::value;
+                dvx = div3<E>(n1_1 - n1_0, sel(ks, xq0.hf, fx0), s6 - s6_jm, hy_n, s5 - sel(ks, s5_km, R(0)), hz_n);
+                dvy = div3<E>(s6 - s6_m, gx, n2_0_jp - n2_0, uy_g2, s4 - sel(ks, s4_km, R(0)), hz_n);
+                dvz = div3<E>(s5 - s5_m, gx, s4 - s4_jm, hy_n, n3_0_kp - n3_0, uz_g3);
+            };
+            if (QUOT && (far | far_m)) divergence(std::integral_constant<int, 1>());
+            else divergence(std::integral_constant<int, EXACT>());
             const unsigned soff = uni((unsigned)i * plane * (unsigned)sizeof(R));
             const unsigned slo = uni((unsigned)i * plane * (unsigned)sizeof(lo_t));
             // lo parts decoded against their stored hi (c0 is the stored
@@ -441,31 +484,24 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
             const R ol1 = COMP ? lo_decode(oin.o1, oin.ol1) : R(0);
             const R ol2 = COMP ? lo_decode(oin.o2, oin.ol2) : R(0);
             const bool wall = !FX && i == 0;  // uy, uz on the x = 0 wall stay 0
-            // ux (base_solver.py:441-447, 495-501)
             {
-                const R dv = div3<EXACT>(n1_1 - n1_0, sel(ks, xq0.hf, m.fx0), s6 - s6_jm, hy_n,
-                                         s5 - sel(ks, s5_km, R(0)), hz_n);
                 const V<R> cur = {c0.x, cl0};
-                const V<R> s0 = leap_from<MODE, SPONGE>(cur, oin.o0, ol0, mget(smat, c1.id, M_COEF), dv, s);
+                const V<R> s0 = leap_from<MODE, SPONGE>(cur, oin.o0, ol0, mget(smat, c1.id, M_COEF), dvx, s);
                 const V<R> above = {ux0_kp, COMP ? above0(cl0) : R(0)};
                 if (wx && (FX || i <= m.nx - 3))
                     put_tile<0, MODE>(m, bf, boff, loff, soff, slo, top_xy, s0, cur, above);
             }
-            // uy (base_solver.py:449-455, 503-509)
             {
-                const R dv = div3<EXACT>(s6 - s6_m, gx, n2_0_jp - n2_0, uy_g2, s4 - sel(ks, s4_km, R(0)), hz_n);
                 const V<R> cur = {c0.y, cl1};
-                V<R> s0 = leap_from<MODE, SPONGE>(cur, oin.o1, ol1, mget(smat, id_jp, M_COEF), dv, s);
+                V<R> s0 = leap_from<MODE, SPONGE>(cur, oin.o1, ol1, mget(smat, id_jp, M_COEF), dvy, s);
                 if (wall) s0 = {R(0), R(0)};
                 const V<R> above = {uy0_kp, COMP ? above0(cl1) : R(0)};
                 if (wy && (FX || i <= m.nx - 2))
                     put_tile<1, MODE>(m, bf, boff, loff, soff, slo, top_xy, s0, cur, above);
             }
-            // uz (base_solver.py:457-463, 511-517)
             {
-                const R dv = div3<EXACT>(s5 - s5_m, gx, s4 - s4_jm, hy_n, n3_0_kp - n3_0, uz_g3);
                 const V<R> cur = {c0.z, cl2};
-                V<R> s0 = leap_from<MODE, SPONGE>(cur, oin.o2, ol2, mget(smat, ks ? id_kp : c0.id, M_COEF), dv, s);
+                V<R> s0 = leap_from<MODE, SPONGE>(cur, oin.o2, ol2, mget(smat, ks ? id_kp : c0.id, M_COEF), dvz, s);
                 if (wall) s0 = {R(0), R(0)};
                 const V<R> above = {above0(c0.z), COMP ? above0(cl2) : R(0)};
                 if (wz && (FX || i <= m.nx - 2))
@@ -479,6 +515,7 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
         n3_0 = n3_1;
         s5_m = s5;
         s6_m = s6;
+        far_m = far;
     };
 
     // planes ib-1, ib+1, ... use parity 0 for plane i+1; ib, ib+2, ... parity 1
@@ -497,8 +534,10 @@ PF_DEV void tiled_march(const Mesh<R>& m, TiledLds<R, TJ, KZ>& L, int kl, int ro
 // 0).  Every thread of the block calls it; it ends without a barrier, so a
 // caller that reuses L for another tile syncs first.
 template <class R, int MODE, bool SPONGE, int TJ, int KZ>
-PF_DEV void tiled_tile(const Mesh<R>& m, const TileMap& tm, int t, TiledLds<R, TJ, KZ>& L, int jstep = TJ - 2,
-                       int x0 = 0) {
+PF_DEV void tiled_tile(const Mesh<R>& m, const TileMap& tm, int t, TiledLds<R, TJ, KZ, Spacing<R, MODE>>& L,
+                       int jstep = TJ - 2, int x0 = 0) {
+    typedef Spacing<R, MODE> H;
+    constexpr bool QUOT = MODE == MODE_FP64Q;
     const int kl = threadIdx.x % KZ;
     const int row = threadIdx.y * (64 / KZ) + threadIdx.x / KZ;
     const int kt = t % tm.nkt;
@@ -517,9 +556,10 @@ PF_DEV void tiled_tile(const Mesh<R>& m, const TileMap& tm, int t, TiledLds<R, T
     for (int e = tid; e < m.nmat * MAT_STRIDE; e += TJ * KZ) L.smat[e] = m.mat[e];
     for (int e = tid; e < ie - ib + 3; e += TJ * KZ) {
         const int p = ib - 1 + e;
-        XPlane<R> x;
-        x.hs = (p >= 1 && p <= m.nx - 2) ? m.sx[p - 1] : R(1);
-        x.hf = (p >= 0 && p <= m.nx - 2) ? m.fx[p] : R(1);
+        XPlane<R, H> x;
+        const bool in = p >= 1 && p <= m.nx - 2, ih = p >= 0 && p <= m.nx - 2;
+        x.hs = spacing<H>(in ? m.sx[p - 1] : R(1), QUOT && in ? m.rsx[p - 1] : R(1));
+        x.hf = spacing<H>(ih ? m.fx[p] : R(1), QUOT && ih ? m.rfx[p] : R(1));
         x.dp = (SPONGE && p >= 0 && p < m.nx) ? m.dpx[p] : R(0);
         x.pad = R(0);
         L.sxp[e] = x;
@@ -540,8 +580,8 @@ PF_DEV void tiled_tile(const Mesh<R>& m, const TileMap& tm, int t, TiledLds<R, T
 // KZ lanes along z per tile row (64: one row per wavefront; 32: two rows
 // per wavefront, lanes 0-31 and 32-63), TJ rows along y per block.
 template <class R, int MODE, bool SPONGE, int TJ, int KZ>
-__global__ __launch_bounds__(TJ * KZ, (MODE == MODE_FP32 ? 4 : 2)) void k_sweep_tiled(Mesh<R> m, TileMap tm) {
-    __shared__ TiledLds<R, TJ, KZ> L;
+__global__ __launch_bounds__(TJ * KZ, (MODE == MODE_FP32 ? 4 : MODE == MODE_FP64Q ? 3 : 2)) void k_sweep_tiled(Mesh<R> m, TileMap tm) {
+    __shared__ TiledLds<R, TJ, KZ, Spacing<R, MODE>> L;
     tiled_tile<R, MODE, SPONGE, TJ, KZ>(m, tm, xcd_remap((int)blockIdx.x, (int)gridDim.x), L);
 }
 
