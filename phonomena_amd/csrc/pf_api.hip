@@ -617,22 +617,6 @@ static int launch_sweep_t(const pf_ctx* c, const Mesh<R>& m, hipStream_t s) {
     }
 }
 
-template <class R>
-static int launch_probe_t(const pf_ctx* c, const Mesh<R>& m, hipStream_t s) {
-    if (c->probe[2] <= 0) return PF_OK;
-    // a step index known on the host (no device counter): launch only on
-    // the steps that record a frame (the kernel checks it again)
-    if (!m.step_base && (m.step_off >= m.nsteps || (m.step_off + 1) % c->every != 0)) return PF_OK;
-    // newest level after this step = the n* buffers of the view
-    const int pts = c->probe[2] * c->probe[5];
-    hipLaunchKernelGGL((k_probe<R>), dim3((unsigned)((pts + 255) / 256)), dim3(256), 0, s, (const R*)m.n2,
-                       (const lo_t*)m.nl2, c->plane, c->pz, c->probe[0], c->probe[1], c->probe[2], c->probe[3],
-                       c->probe[4], c->probe[5], c->ring, c->cap, c->d_frame, (int*)(c->d_frame + 1),
-                       m.step_base, m.step_off, c->every, m.nsteps);
-    HIPCHK(hipGetLastError());
-    return PF_OK;
-}
-
 // Whether the step of view m records a probe frame: always possibly when its
 // step index is on the device (the kernel decides), else by the host index.
 template <class R>
@@ -641,30 +625,24 @@ static bool probe_due(const pf_ctx* c, const Mesh<R>& m) {
     return m.step_base || (m.step_off < m.nsteps && (m.step_off + 1) % c->every == 0);
 }
 
-// The faces of the level view m writes, and the step's probe frame: one
-// launch with the row-wise face kernel, which takes the probe blocks too;
-// the per-cell face kernel and a probe launch on meshes too small for it.
+// The faces of the level view m writes, and the step's probe frame, in one
+// launch.
 template <class R, int MODE>
 static int launch_faces_probe_t(const pf_ctx* c, const Mesh<R>& m, hipStream_t s) {
     long long rb, eb;
-    if (face_rows_grid(c->nx, c->ny, c->nz, rb, eb)) {
-        FaceProbe pr = {};
-        pr.every = 1;
-        if (probe_due(c, m)) {
-            const int* q = c->probe;
-            pr = {c->ring, c->d_frame, (int*)(c->d_frame + 1), q[0], q[1], q[2], q[3], q[4], q[5], c->cap, c->every,
-                  (q[2] * q[5] + 255) / 256};
-        }
-        if (rb + eb + pr.blocks > 0x7fffffffLL) return fail(PF_ERR_ARG, "too many face cells");
-        hipLaunchKernelGGL((k_faces_rows<R, MODE>), dim3((unsigned)(rb + eb + pr.blocks)), dim3(256), 0, s, m, (int)rb,
-                           (int)eb, pr);
-        HIPCHK(hipGetLastError());
-        return PF_OK;
+    face_rows_grid(c->nx, c->ny, c->nz, rb, eb);
+    FaceProbe pr = {};
+    pr.every = 1;
+    if (probe_due(c, m)) {
+        const int* q = c->probe;
+        pr = {c->ring, c->d_frame, (int*)(c->d_frame + 1), q[0], q[1], q[2], q[3], q[4], q[5], c->cap, c->every,
+              (q[2] * q[5] + 255) / 256};
     }
-    const long long n = face_total(c->nx, c->ny, c->nz);
-    hipLaunchKernelGGL((k_faces<R, MODE>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m, n);
+    if (rb + eb + pr.blocks > 0x7fffffffLL) return fail(PF_ERR_ARG, "too many face cells");
+    hipLaunchKernelGGL((k_faces_rows<R, MODE>), dim3((unsigned)(rb + eb + pr.blocks)), dim3(256), 0, s, m, (int)rb,
+                       (int)eb, pr);
     HIPCHK(hipGetLastError());
-    return launch_probe_t<R>(c, m, s);
+    return PF_OK;
 }
 
 // The view a sweep of MODE reads: with MODE_FP64P the spacing tables and

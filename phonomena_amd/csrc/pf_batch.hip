@@ -1,17 +1,18 @@
 // Batched stepping: many contexts of one precision stepped together.
 //
-// Per step the batch issues three launches whatever its size:
+// Per step the batch issues two launches whatever its size:
 //   1. one persistent sweep over a combined tile work-list of all members
 //      (the same per-tile code as the single-mesh tiled sweep, so a member's
 //      fields are bit-identical to stepping it alone);
-//   2. one launch over all members' boundary-face cells;
-//   3. one launch recording every member's probe frame, whose last block to
-//      finish advances every member's device step counter.
-// The step index of a member lives on the device, and which of its two
-// levels is current follows from it, so K steps are captured once in a HIP
-// graph and replayed.  A member whose step counter reaches its source-table
-// length (its step budget) stops: its tiles, faces and probes return at
-// once and its counter no longer moves.
+//   2. one launch over all members' boundary-face cells, which records their
+//      probe frames too.
+// The steps since the tables were built are counted on the device (a launch
+// takes its place in a group of steps as an argument, and one small launch
+// per group moves the counters on), and which of a member's two levels is
+// current follows from that, so K steps are captured once in a HIP graph and
+// replayed.  A member whose step index reaches its source-table length (its
+// step budget) stops: its tiles, faces and probes return at once and its
+// counters no longer move.
 //
 // Work-list: the tiles of every member, member after member in tile order,
 // cut into 8 contiguous runs of equal plane count, one per XCD (the device
@@ -44,13 +45,9 @@ struct BMember {
     Mesh<R> view[2];        // mesh views with level 0 / level 1 current
     TileMap tm;
     long long* step;        // the member's device step counter
-    long long t0;           // its step count when the views were taken
-    int cur0;               // and its current level then
-    int probe[6];
-    int every, cap;
-    double* ring;
-    long long* frame;
-    long long faces;        // boundary-face cells per step
+    long long t0;           // its step count when the views were taken (view[0])
+    FaceProbe probe;        // ni = 0: none
+    int row_blocks, edge_blocks;  // as face_rows_grid gives them
     long long budget;       // source-table length
 };
 
@@ -80,25 +77,36 @@ PF_DEV T load_const(const T* p) {
     return v;
 }
 
-// Mesh view of member i at its current step (the step counter is written
-// only between launches, so one read per block is current for the launch).
+// Pointers read from memory lead to global memory, as the compiler knows of a
+// kernel's arguments; otherwise it accesses them with flat instructions, which
+// wait for the LDS too.
+template <class... P>
+PF_DEV void in_global(P&... p) {
+    ((p = (P)(__attribute__((address_space(1))) std::remove_reference_t<decltype(*p)>*)(uintptr_t)p), ...);
+}
+
+// Mesh view of member i, n steps after the tables were built.
 template <class R>
-PF_DEV Mesh<R> current_view(const BMember<R>* mem, int i) {
+PF_DEV Mesh<R> current_view(const BMember<R>* mem, int i, long long n) {
     CMember<R>* cm = (CMember<R>*)mem;
-    const long long tt = *cm[i].step;
-    const int p = cm[i].cur0 ^ (int)((tt - cm[i].t0) & 1);
-    return load_const(&mem[i].view[p]);
+    Mesh<R> m = load_const(&mem[i].view[n & 1]);
+    m.step_base = nullptr;
+    m.step_off = cm[i].t0 + n;
+    in_global(m.c0, m.c1, m.c2, m.cl0, m.cl1, m.cl2, m.n0, m.n1, m.n2, m.nl0, m.nl1, m.nl2, m.wave, m.mat, m.sx, m.fx,
+              m.sy, m.fy, m.sz, m.fz, m.dpx, m.dpy, m.dpz);
+    return m;
 }
 
 template <class R, int MODE, bool SPONGE, int TJ, int KZ>
 __global__ __launch_bounds__(TJ * KZ, (MODE == MODE_FP32 ? 4 : 2)) void k_batch_sweep(
     const BMember<R>* __restrict__ mem, const WorkItem* __restrict__ items, const int* __restrict__ qbeg,
-    int* __restrict__ ctr, const long long* __restrict__ bstep) {
+    int* __restrict__ ctr, const long long* __restrict__ bstep, int off) {
     __shared__ TiledLds<R, TJ, KZ> L;
     __shared__ int s_item;
     const int tid = threadIdx.y * 64 + threadIdx.x;
     const int x = (int)(blockIdx.x % NXCD);
-    const int par = (int)(*bstep & 1);
+    const long long n = *bstep + off;
+    const int par = (int)(n & 1);
     if (blockIdx.x == 0 && tid < NXCD) ctr[(par ^ 1) * NXCD + tid] = 0;  // next step's counters
     int* c = ctr + par * NXCD + x;
     const int end = qbeg[x + 1];
@@ -112,63 +120,78 @@ __global__ __launch_bounds__(TJ * KZ, (MODE == MODE_FP32 ? 4 : 2)) void k_batch_
         const int mi = ci[it].member, tile = ci[it].tile;
         CMember<R>* cm = (CMember<R>*)mem;
         const TileMap tm = {cm[mi].tm.nkt, cm[mi].tm.njt, cm[mi].tm.nxc, cm[mi].tm.xchunk};
-        const Mesh<R> m = current_view(mem, mi);
+        const Mesh<R> m = current_view(mem, mi, n);
         tiled_tile<R, MODE, SPONGE, TJ, KZ>(m, tm, tile, L);
     }
 }
 
 // Face block g of a batched step: its member and its index among that
-// member's face blocks (one table load instead of a search).
+// member's blocks (one table load instead of a search).
 struct FaceBlock {
     int member, block;
 };
 
-// Face cells of all members, BATCH_FACE_CELLS per block (four per thread).
-constexpr int BATCH_FACE_CELLS = 1024;
-template <class R, int MODE>
-__global__ __launch_bounds__(256) void k_batch_faces(const BMember<R>* __restrict__ mem,
-                                                     const FaceBlock* __restrict__ fmap) {
-    const FaceBlock fb = load_const(&fmap[blockIdx.x]);
-    CMember<R>* cm = (CMember<R>*)mem;
-    const Mesh<R> m = current_view(mem, fb.member);
-    faces_run<R, MODE, BATCH_FACE_CELLS / 256>(m, (long long)fb.block * BATCH_FACE_CELLS, cm[fb.member].faces);
+// Blocks of member c's face cells and probe points.
+template <class R>
+int face_blocks(BMember<R>& e, const pf_ctx* c) {
+    const int* q = c->probe;
+    e.probe = {c->ring, c->d_frame, nullptr, q[0], q[1], q[2], q[3], q[4], q[5], c->cap, c->every,
+               q[2] > 0 ? (q[2] * q[5] + 255) / 256 : 0};
+    long long rb, eb;
+    face_rows_grid(c->nx, c->ny, c->nz, rb, eb);
+    e.row_blocks = (int)rb;
+    e.edge_blocks = (int)eb;
+    return (int)(rb + eb) + e.probe.blocks;
 }
 
-// Block i records member i's probe frame.  Every block then counts itself
-// done; the last one (which sees every other block's count, and so every
-// block's reads of its step counter, before it) advances all members' step
-// counters, the batch's step parity, and resets the count for the next
-// step.  No block waits for another.
+// Face cells and probe frames of all members: every block does what a block
+// of k_faces_rows does for one mesh.  It is bound by its fixed cost and the
+// chain of loads each wave makes (member, view, cells): 14.7 us at 16 members
+// of 14.2 M nodes in FP32C, against 24.7 us with 1024 cells of a flat list per
+// block and 6.0 us for the frames and the counters in a launch of their own;
+// a step of 5 members of 1.4 M nodes went from 64 to 49 us.
+template <class R, int MODE>
+__global__ __launch_bounds__(256) void k_batch_faces(const BMember<R>* __restrict__ mem,
+                                                     const FaceBlock* __restrict__ fmap,
+                                                     const long long* __restrict__ bstep, int off) {
+    const long long n = *bstep + off;
+    const FaceBlock fb = load_const(&fmap[blockIdx.x]);
+    CMember<R>& e = ((CMember<R>*)mem)[fb.member];
+    const auto& v = e.view[n & 1];
+    const long long tt = e.t0 + n;
+    if (tt >= v.nsteps) return;
+    const R w = (R)v.wave[tt];
+    const int rows = e.row_blocks, edges = e.edge_blocks;
+    // each branch takes the view by itself: what it does not use is then not
+    // loaded (one view for all was 250 scalar registers more than there are)
+    auto view = [&]() { return current_view(mem, fb.member, n); };
+    if (fb.block < rows) {
+        face_rows_block<R, MODE>(v.nx, v.ny, v.nz, view, fb.block, w);
+        return;
+    }
+    if (fb.block < rows + edges) {
+        face_edges_block<R, MODE>(view(), fb.block - rows, w);
+        return;
+    }
+    const FaceProbe pr = load_const(&mem[fb.member].probe);
+    if ((tt + 1) % pr.every != 0) return;
+    const int p = (fb.block - rows - edges) * 256 + (int)threadIdx.x, np = pr.ni * pr.nj;
+    if (p < np) pr.ring[(tt / pr.every) % pr.cap * np + p] = probe_point<R, MODE>(view(), pr, p, w);
+}
+
+// The counters after a group of `by` steps.  A member's frames are those its
+// steps have recorded.
 template <class R>
-__global__ __launch_bounds__(256) void k_batch_probe(const BMember<R>* __restrict__ mem,
-                                                     long long* const* __restrict__ steps,
-                                                     const long long* __restrict__ budget, int nmem,
-                                                     long long* __restrict__ bstep, int* __restrict__ done) {
-    __shared__ int s_last;
+__global__ __launch_bounds__(256) void k_batch_advance(const BMember<R>* __restrict__ mem, int nmem,
+                                                       long long* __restrict__ bstep, int by) {
     CMember<R>* cm = (CMember<R>*)mem;
-    const int i = (int)blockIdx.x;
-    if (cm[i].probe[2] > 0) {
-        const Mesh<R> m = current_view(mem, i);
-        probe_record<R>(m.n2, m.nl2, m.plane, m.pz, cm[i].probe[0], cm[i].probe[1], cm[i].probe[2],
-                        cm[i].probe[3], cm[i].probe[4], cm[i].probe[5], cm[i].ring, cm[i].cap, cm[i].frame,
-                        *cm[i].step, cm[i].every, cm[i].budget);
+    for (int i = threadIdx.x; i < nmem; i += 256) {
+        const long long v = *cm[i].step + by, cap = cm[i].budget;
+        const long long t = v < cap ? v : cap;
+        *cm[i].step = t;
+        if (cm[i].probe.blocks > 0) *cm[i].probe.frame = t / cm[i].probe.every;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        s_last = atomicAdd(done, 1) == nmem - 1;
-    }
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
-    for (int k = threadIdx.x; k < nmem; k += blockDim.x) {
-        const long long v = *steps[k] + 1;
-        *steps[k] = v < budget[k] ? v : budget[k];
-    }
-    if (threadIdx.x == 0) {
-        *bstep += 1;
-        *done = 0;
-    }
+    if (threadIdx.x == 0) *bstep += by;
 }
 
 }  // namespace pf
@@ -191,9 +214,6 @@ struct pf_batch {
     long long* d_bstep = nullptr;
     FaceBlock* d_fmap = nullptr;
     size_t fmap_cap = 0;
-    long long** d_steps = nullptr;
-    long long* d_budget = nullptr;
-    size_t nmem_cap = 0;
     long long face_blocks = 0;
     int grid = 0;
     bool dirty = true;
@@ -217,10 +237,9 @@ int free_graph(pf_batch* b) {
 void free_tables(pf_batch* b) {
     auto F = [](void* p) { if (p) (void)hipFree(p); };
     F(b->d_mem); F(b->d_items); F(b->d_qbeg); F(b->d_ctr); F(b->d_bstep); F(b->d_fmap);
-    F(b->d_steps); F(b->d_budget);
     b->d_mem = nullptr; b->d_items = nullptr; b->d_qbeg = nullptr; b->d_ctr = nullptr; b->d_bstep = nullptr;
-    b->d_fmap = nullptr; b->d_steps = nullptr; b->d_budget = nullptr;
-    b->mem_bytes = b->items_cap = b->nmem_cap = b->fmap_cap = 0;
+    b->d_fmap = nullptr;
+    b->mem_bytes = b->items_cap = b->fmap_cap = 0;
 }
 
 // Default rows x lanes of a batch (the autotuner refines them): 16 x 32, 8 x
@@ -304,8 +323,6 @@ int build_t(pf_batch* b) {
     std::vector<WorkItem> items;
     std::vector<long long> cost;  // planes per work item
     std::vector<long long> fblk((size_t)nmem + 1, 0);
-    std::vector<long long*> steps((size_t)nmem);
-    std::vector<long long> budget((size_t)nmem);
     for (int i = 0; i < nmem; i++) {
         pf_ctx* c = b->members[(size_t)i];
         BMember<R>& e = mem[(size_t)i];
@@ -313,23 +330,12 @@ int build_t(pf_batch* b) {
         // view[0]: the level current now; view[1]: after an odd count of steps
         e.view[0] = make_view<R>(c, c->cur, c->old, c->old);
         e.view[1] = make_view<R>(c, c->old, c->cur, c->cur);
-        for (int p = 0; p < 2; p++) {
-            e.view[p].step_base = c->d_step;
-            e.view[p].step_off = 0;
-        }
         // planes per chunk: about tx, evened out over the mesh
         const int nch = (c->nx + tx - 1) / tx;
         const int xchunk = std::min((c->nx + nch - 1) / nch, XT - 3);
         e.tm = tile_map(c, tj, tz, xchunk);
         e.step = c->d_step;
         e.t0 = c->step;
-        e.cur0 = 0;
-        for (int q = 0; q < 6; q++) e.probe[q] = c->probe[q];
-        e.every = c->every;
-        e.cap = c->cap;
-        e.ring = c->ring;
-        e.frame = c->d_frame;
-        e.faces = face_total(c->nx, c->ny, c->nz);
         e.budget = c->wave_len;
         const long long nt = (long long)e.tm.nkt * e.tm.njt * e.tm.nxc;
         for (long long t = 0; t < nt; t++) {
@@ -338,9 +344,7 @@ int build_t(pf_batch* b) {
             const int ib = xc * e.tm.xchunk;
             cost.push_back(std::min(e.tm.xchunk, c->nx - ib) + 2);
         }
-        fblk[(size_t)i + 1] = fblk[(size_t)i] + (e.faces + BATCH_FACE_CELLS - 1) / BATCH_FACE_CELLS;
-        steps[(size_t)i] = c->d_step;
-        budget[(size_t)i] = c->wave_len;
+        fblk[(size_t)i + 1] = fblk[(size_t)i] + face_blocks(e, c);
     }
     if (items.size() > 0x7fffffff) return fail(PF_ERR_ARG, "batch work-list too long");
     if (fblk[(size_t)nmem] > 0x7fffffffLL) return fail(PF_ERR_ARG, "batch has too many face cells");
@@ -365,21 +369,18 @@ int build_t(pf_batch* b) {
     }
     // (re)allocate and upload
     const size_t mb = sizeof(BMember<R>) * (size_t)nmem;
-    if (b->mem_bytes < mb || b->items_cap < items.size() || b->nmem_cap < (size_t)nmem || b->fmap_cap < fmap.size() ||
+    if (b->mem_bytes < mb || b->items_cap < items.size() || b->fmap_cap < fmap.size() ||
         !b->d_qbeg) {
         free_tables(b);
         HIPCHK(hipMalloc(&b->d_mem, mb));
         HIPCHK(hipMalloc((void**)&b->d_items, sizeof(WorkItem) * std::max<size_t>(items.size(), 1)));
         HIPCHK(hipMalloc((void**)&b->d_qbeg, sizeof(int) * (NXCD + 1)));
-        // two steps' queue counters, then the probe launch's done count
-        HIPCHK(hipMalloc((void**)&b->d_ctr, sizeof(int) * (2 * NXCD + 1)));
+        // two steps' queue counters
+        HIPCHK(hipMalloc((void**)&b->d_ctr, sizeof(int) * (2 * NXCD)));
         HIPCHK(hipMalloc((void**)&b->d_bstep, sizeof(long long)));
         HIPCHK(hipMalloc((void**)&b->d_fmap, sizeof(FaceBlock) * std::max<size_t>(fmap.size(), 1)));
-        HIPCHK(hipMalloc((void**)&b->d_steps, sizeof(long long*) * (size_t)nmem));
-        HIPCHK(hipMalloc((void**)&b->d_budget, sizeof(long long) * (size_t)nmem));
         b->mem_bytes = mb;
         b->items_cap = std::max<size_t>(items.size(), 1);
-        b->nmem_cap = (size_t)nmem;
         b->fmap_cap = std::max<size_t>(fmap.size(), 1);
     }
     HIPCHK(hipStreamSynchronize(b->stream));
@@ -387,12 +388,10 @@ int build_t(pf_batch* b) {
     if (!items.empty())
         HIPCHK(hipMemcpy(b->d_items, items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(b->d_qbeg, qbeg.data(), sizeof(int) * (NXCD + 1), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(b->d_ctr, 0, sizeof(int) * (2 * NXCD + 1)));
+    HIPCHK(hipMemset(b->d_ctr, 0, sizeof(int) * (2 * NXCD)));
     HIPCHK(hipMemset(b->d_bstep, 0, sizeof(long long)));
     if (!fmap.empty())
         HIPCHK(hipMemcpy(b->d_fmap, fmap.data(), sizeof(FaceBlock) * fmap.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(b->d_steps, steps.data(), sizeof(long long*) * (size_t)nmem, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(b->d_budget, budget.data(), sizeof(long long) * (size_t)nmem, hipMemcpyHostToDevice));
     for (int i = 0; i < nmem; i++) {
         pf_ctx* c = b->members[(size_t)i];
         HIPCHK(hipMemcpy(c->d_step, &c->step, sizeof(long long), hipMemcpyHostToDevice));
@@ -412,44 +411,45 @@ int build(pf_batch* b) {
 }
 
 template <class R, int MODE, bool SPONGE, int TJ, int KZ>
-void launch_sweep(pf_batch* b) {
+void launch_sweep(pf_batch* b, int off) {
     hipLaunchKernelGGL((k_batch_sweep<R, MODE, SPONGE, TJ, KZ>), dim3((unsigned)b->grid), dim3(64, TJ * KZ / 64), 0,
                        b->stream, (const BMember<R>*)b->d_mem, (const WorkItem*)b->d_items, (const int*)b->d_qbeg,
-                       b->d_ctr, (const long long*)b->d_bstep);
+                       b->d_ctr, (const long long*)b->d_bstep, off);
 }
 
 template <class R, int MODE, bool SPONGE>
-void launch_sweep_s(pf_batch* b, int tj, int tz) {
-    if (tz == 64 && tj == 16) launch_sweep<R, MODE, SPONGE, 16, 64>(b);
-    else if (tz == 64 && tj == 8) launch_sweep<R, MODE, SPONGE, 8, 64>(b);
-    else if (tz == 32 && tj == 32) launch_sweep<R, MODE, SPONGE, 32, 32>(b);
-    else if (tz == 32 && tj == 16) launch_sweep<R, MODE, SPONGE, 16, 32>(b);
-    else launch_sweep<R, MODE, SPONGE, 8, 32>(b);
+void launch_sweep_s(pf_batch* b, int tj, int tz, int off) {
+    if (tz == 64 && tj == 16) launch_sweep<R, MODE, SPONGE, 16, 64>(b, off);
+    else if (tz == 64 && tj == 8) launch_sweep<R, MODE, SPONGE, 8, 64>(b, off);
+    else if (tz == 32 && tj == 32) launch_sweep<R, MODE, SPONGE, 32, 32>(b, off);
+    else if (tz == 32 && tj == 16) launch_sweep<R, MODE, SPONGE, 16, 32>(b, off);
+    else launch_sweep<R, MODE, SPONGE, 8, 32>(b, off);
 }
 
-// Issue one batched step (three launches) on the batch stream.
+// Issue a group of k batched steps on the batch stream: two launches a step
+// and the one that moves the counters on.
 template <class R, int MODE>
-int issue_step_t(pf_batch* b) {
+int issue_steps_t(pf_batch* b, int k) {
     int tj, tz;
     batch_shape(b, tj, tz);
-    const int nmem = (int)b->members.size();
-    if (b->sponge == 1) launch_sweep_s<R, MODE, true>(b, tj, tz);
-    else launch_sweep_s<R, MODE, false>(b, tj, tz);
-    if (b->face_blocks > 0)
-        hipLaunchKernelGGL((k_batch_faces<R, MODE>), dim3((unsigned)b->face_blocks), dim3(256), 0, b->stream,
-                           (const BMember<R>*)b->d_mem, (const FaceBlock*)b->d_fmap);
-    hipLaunchKernelGGL((k_batch_probe<R>), dim3((unsigned)nmem), dim3(256), 0, b->stream, (const BMember<R>*)b->d_mem,
-                       (long long* const*)b->d_steps, (const long long*)b->d_budget, nmem, b->d_bstep,
-                       b->d_ctr + 2 * NXCD);
+    const BMember<R>* mem = (const BMember<R>*)b->d_mem;
+    for (int off = 0; off < k; off++) {
+        if (b->sponge == 1) launch_sweep_s<R, MODE, true>(b, tj, tz, off);
+        else launch_sweep_s<R, MODE, false>(b, tj, tz, off);
+        hipLaunchKernelGGL((k_batch_faces<R, MODE>), dim3((unsigned)b->face_blocks), dim3(256), 0, b->stream, mem,
+                           (const FaceBlock*)b->d_fmap, (const long long*)b->d_bstep, off);
+    }
+    hipLaunchKernelGGL((k_batch_advance<R>), dim3(1), dim3(256), 0, b->stream, mem, (int)b->members.size(), b->d_bstep,
+                       k);
     HIPCHK(hipGetLastError());
     return PF_OK;
 }
 
-int issue_step(pf_batch* b) {
+int issue_steps(pf_batch* b, int k) {
     switch (b->precision) {
-        case PF_FP64: return issue_step_t<double, MODE_FP64>(b);
-        case PF_FP32: return issue_step_t<float, MODE_FP32>(b);
-        default: return issue_step_t<float, MODE_FP32C>(b);
+        case PF_FP64: return issue_steps_t<double, MODE_FP64>(b, k);
+        case PF_FP32: return issue_steps_t<float, MODE_FP32>(b, k);
+        default: return issue_steps_t<float, MODE_FP32C>(b, k);
     }
 }
 
@@ -458,7 +458,7 @@ int capture(pf_batch* b, int k) {
     int rc = free_graph(b);
     if (rc) return rc;
     HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    for (int s = 0; s < k && !rc; s++) rc = issue_step(b);
+    rc = issue_steps(b, k);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (rc) {
@@ -496,8 +496,8 @@ int step_n(pf_batch* b, long long n) {
         if (b->graph_steps != GRAPH_STEPS && (rc = capture(b, GRAPH_STEPS))) return rc;
         for (; done + GRAPH_STEPS <= n; done += GRAPH_STEPS) HIPCHK(hipGraphLaunch(b->exec, b->stream));
     }
-    for (; done < n; done++)
-        if ((rc = issue_step(b))) return rc;
+    for (; done < n; done += std::min<long long>(n - done, GRAPH_STEPS))
+        if ((rc = issue_steps(b, (int)std::min<long long>(n - done, GRAPH_STEPS)))) return rc;
     account(b, n);
     return PF_OK;
 }

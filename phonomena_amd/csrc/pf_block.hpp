@@ -16,8 +16,8 @@
 //
 // What bounds it: the launch (about 4 us with its loads and stores) and the
 // chain of T steps; block_map weighs the nodes computed twice against the
-// launches saved.  The faces take a pass per axis over values in LDS; as the
-// recursive chain of final_value they cost twice the step (one step of
+// launches saved.  The faces take a pass per axis over values in LDS; as a
+// recursion over the faces a cell lies on they cost twice the step (one step of
 // 31 x 21 x 6 nodes in FP64 with divisions 9.9 against 7.4 us a launch).
 //
 // The values are those of the sweep and the face kernels, bit for bit: the

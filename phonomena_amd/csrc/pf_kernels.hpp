@@ -248,17 +248,6 @@ PF_DEV V<R> cur_q(const Mesh<R>& m, int i, int j, int k, R w) {
     return v;
 }
 
-template <int Q, class R>
-PF_DEV V<R> new_q(const Mesh<R>& m, int i, int j, int k) {
-    long long id = at(m, i, j, k);
-    const R* n = Q == 0 ? m.n0 : (Q == 1 ? m.n1 : m.n2);
-    const lo_t* nl = Q == 0 ? m.nl0 : (Q == 1 ? m.nl1 : m.nl2);
-    V<R> v;
-    v.h = n[id];
-    v.l = nl ? lo_decode(v.h, nl[id]) : R(0);
-    return v;
-}
-
 // a + c * (b - d), the reference's `q[..] + c*(q_new[..] - q[..])`
 template <int MODE, class R>
 PF_DEV V<R> mur_map(V<R> a, R ch, R cl, V<R> b, V<R> d) {
@@ -270,42 +259,6 @@ PF_DEV V<R> mur_map(V<R> a, R ch, R cl, V<R> b, V<R> d) {
         r.l = R(0);
     }
     return r;
-}
-
-// Value after stage I and the x = max face (face index 0).
-template <int Q, int MODE, class R>
-PF_DEV V<R> after_x(const Mesh<R>& m, int i, int j, int k, R w) {
-    const int Lx = Ext<Q>::Lx(m.nx);
-    if (i == Lx)
-        return mur_map<MODE>(cur_q<Q>(m, Lx - 1, j, k, w), m.mur[0 + Q], m.mur_lo[0 + Q],
-                             new_q<Q>(m, Lx - 1, j, k), cur_q<Q>(m, Lx, j, k, w));
-    return new_q<Q>(m, i, j, k);
-}
-// ... then the y = 0 face (face index 1)
-template <int Q, int MODE, class R>
-PF_DEV V<R> after_y0(const Mesh<R>& m, int i, int j, int k, R w) {
-    if (j == 0)
-        return mur_map<MODE>(cur_q<Q>(m, i, 1, k, w), m.mur[3 + Q], m.mur_lo[3 + Q],
-                             after_x<Q, MODE>(m, i, 1, k, w), cur_q<Q>(m, i, 0, k, w));
-    return after_x<Q, MODE>(m, i, j, k, w);
-}
-// ... then the y = max face (face index 2)
-template <int Q, int MODE, class R>
-PF_DEV V<R> after_y1(const Mesh<R>& m, int i, int j, int k, R w) {
-    const int Ly = Ext<Q>::Ly(m.ny);
-    if (j == Ly)
-        return mur_map<MODE>(cur_q<Q>(m, i, Ly - 1, k, w), m.mur[6 + Q], m.mur_lo[6 + Q],
-                             after_y0<Q, MODE>(m, i, Ly - 1, k, w), cur_q<Q>(m, i, Ly, k, w));
-    return after_y0<Q, MODE>(m, i, j, k, w);
-}
-// ... then the z = max face (face index 3): the final value.
-template <int Q, int MODE, class R>
-PF_DEV V<R> final_value(const Mesh<R>& m, int i, int j, int k, R w) {
-    const int Lz = Ext<Q>::Lz(m.nz);
-    if (k == Lz)
-        return mur_map<MODE>(cur_q<Q>(m, i, j, Lz - 1, w), m.mur[9 + Q], m.mur_lo[9 + Q],
-                             after_y1<Q, MODE>(m, i, j, Lz - 1, w), cur_q<Q>(m, i, j, Lz, w));
-    return after_y1<Q, MODE>(m, i, j, k, w);
 }
 
 template <int Q, class R> PF_DEV R* nptr(const Mesh<R>& m) { return Q == 0 ? m.n0 : (Q == 1 ? m.n1 : m.n2); }
@@ -341,124 +294,127 @@ PF_DEV void put_with_zface(const Mesh<R>& m, int i, int j, int k, V<R> s0, V<R> 
 //        (Lx, j, Lz)               0 < j < Ly
 //        (i, 0, Lz), (i, Ly, Lz)   i < Lx
 template <int Q>
-PF_DEV long long face_count(int nx, int ny, int nz) {
-    const long long Lx = Ext<Q>::Lx(nx), Ly = Ext<Q>::Ly(ny), Lz = Ext<Q>::Lz(nz);
-    return (Ly - 1) * Lz + 2 * Lx * Lz + 2 * (Lz + 1) + (Ly - 1) + 2 * Lx;
+PF_DEV int face_edges(int nx, int ny, int nz) {
+    return 2 * (Ext<Q>::Lz(nz) + 1) + Ext<Q>::Ly(ny) - 1 + 2 * Ext<Q>::Lx(nx);
 }
 
+// Box-edge cell t of component Q.
 template <int Q>
-PF_DEV void face_cell(int nx, int ny, int nz, long long t, int& i, int& j, int& k) {
-    const long long Lx = Ext<Q>::Lx(nx), Ly = Ext<Q>::Ly(ny), Lz = Ext<Q>::Lz(nz);
-    long long n = (Ly - 1) * Lz;
-    if (t < n) { i = (int)Lx; j = 1 + (int)(t / Lz); k = (int)(t % Lz); return; }
-    t -= n;
-    n = Lx * Lz;
-    if (t < n) { j = 0; i = (int)(t / Lz); k = (int)(t % Lz); return; }
-    t -= n;
-    if (t < n) { j = (int)Ly; i = (int)(t / Lz); k = (int)(t % Lz); return; }
-    t -= n;
-    if (t < Lz + 1) { i = (int)Lx; j = 0; k = (int)t; return; }
+PF_DEV void face_edge_cell(int nx, int ny, int nz, int t, int& i, int& j, int& k) {
+    const int Lx = Ext<Q>::Lx(nx), Ly = Ext<Q>::Ly(ny), Lz = Ext<Q>::Lz(nz);
+    if (t < Lz + 1) { i = Lx; j = 0; k = t; return; }
     t -= Lz + 1;
-    if (t < Lz + 1) { i = (int)Lx; j = (int)Ly; k = (int)t; return; }
+    if (t < Lz + 1) { i = Lx; j = Ly; k = t; return; }
     t -= Lz + 1;
-    if (t < Ly - 1) { i = (int)Lx; j = 1 + (int)t; k = (int)Lz; return; }
+    if (t < Ly - 1) { i = Lx; j = 1 + t; k = Lz; return; }
     t -= Ly - 1;
-    if (t < Lx) { i = (int)t; j = 0; k = (int)Lz; return; }
-    t -= Lx;
-    i = (int)t; j = (int)Ly; k = (int)Lz;
+    if (t < Lx) { i = t; j = 0; k = Lz; return; }
+    i = t - Lx; j = Ly; k = Lz;
 }
 
+// Final value of a face cell: the interior cell's new value through the Mur
+// maps of the faces it lies on, in the reference's order x = max, y = 0 or
+// y = max, z = max (base_solver.py:525-554), each
+//   face = cur(inside) + c (new(inside) - cur(face)),
+// where inside is the cell one step off that face.  Each map's operands are the
+// level-n values on the way from the interior cell (ii, ji, ki) to the face
+// cell, so five values give all three maps, and their loads leave together
+// (needs Lx >= 1, Ly >= 2, Lz >= 1, so that no step off a face ends on
+// another: meshes have at least four nodes per axis).  As a recursion over the
+// faces the lanes of a wave at different edges took its branches, and their
+// loads, one after another.
 template <int Q, int MODE, class R>
-PF_DEV void face_write(const Mesh<R>& m, long long t, R w) {
-    int i, j, k;
-    face_cell<Q>(m.nx, m.ny, m.nz, t, i, j, k);
-    put<Q, MODE>(m, i, j, k, final_value<Q, MODE>(m, i, j, k, w));
-}
-
-// Face cell t (all three components' cells numbered one after another) of a
-// step whose source value is w.
-template <class R, int MODE>
-PF_DEV void faces_one(const Mesh<R>& m, long long t, R w) {
-    const long long e0 = face_count<0>(m.nx, m.ny, m.nz);
-    const long long e1 = face_count<1>(m.nx, m.ny, m.nz);
-    const long long e2 = face_count<2>(m.nx, m.ny, m.nz);
-    if (t < e0) { face_write<0, MODE>(m, t, w); return; }
-    t -= e0;
-    if (t < e1) { face_write<1, MODE>(m, t, w); return; }
-    t -= e1;
-    if (t < e2) face_write<2, MODE>(m, t, w);
-}
-
-// Face cells [t0, t0 + 256 * PER) of view m, PER per thread of a
-// 256-thread block; the step index and source value are read once.  One
-// mesh's faces run best with one cell per thread (more blocks in flight);
-// the batch, whose blocks first read their member's tables, with four.
-template <class R, int MODE, int PER>
-PF_DEV void faces_run(const Mesh<R>& m, long long t0, long long total) {
-    const long long tt = step_index(m);
-    if (tt >= m.nsteps) return;
-    const R w = (R)m.wave[tt];
-#pragma unroll
-    for (int r = 0; r < PER; r++) {
-        const long long t = t0 + r * 256 + threadIdx.x;
-        if (t < total) faces_one<R, MODE>(m, t, w);
+PF_DEV V<R> face_value(const Mesh<R>& m, int i, int j, int k, R w) {
+    const int Lx = Ext<Q>::Lx(m.nx), Ly = Ext<Q>::Ly(m.ny), Lz = Ext<Q>::Lz(m.nz);
+    const bool fx = i == Lx, fy = j == 0 || j == Ly, fz = k == Lz;
+    const int ii = fx ? Lx - 1 : i, ji = j == 0 ? 1 : (j == Ly ? Ly - 1 : j), ki = fz ? Lz - 1 : k;
+    const R yh = j == 0 ? m.mur[3 + Q] : m.mur[6 + Q], yl = j == 0 ? m.mur_lo[3 + Q] : m.mur_lo[6 + Q];
+    const R* cp = Q == 0 ? m.c0 : (Q == 1 ? m.c1 : m.c2);
+    const R* np = nptr<Q>(m);
+    const long long ia = at(m, ii, ji, ki), ib = at(m, i, ji, ki), ic = at(m, i, j, ki), id = at(m, i, j, k);
+    V<R> v = {np[ia], R(0)}, a = {cp[ia], R(0)}, b = {cp[ib], R(0)}, c = {cp[ic], R(0)}, d = {cp[id], R(0)};
+    if constexpr (MODE == MODE_FP32C) {
+        const lo_t* cl = Q == 0 ? m.cl0 : (Q == 1 ? m.cl1 : m.cl2);
+        const lo_t lv = nlptr<Q>(m)[ia], la = cl[ia], lb = cl[ib], lc = cl[ic], ld = cl[id];
+        v.l = lo_decode(v.h, lv);
+        a.l = lo_decode(a.h, la);
+        b.l = lo_decode(b.h, lb);
+        c.l = lo_decode(c.h, lc);
+        d.l = lo_decode(d.h, ld);
     }
+    if (Q == 2) {  // the source line uz[0, :, 0] reads as w
+        const V<R> src = {w, R(0)};
+        if (ii == 0 && ki == 0) a = src;
+        if (i == 0 && ki == 0) b = c = src;
+        if (i == 0 && k == 0) d = src;
+    }
+    const V<R> x = mur_map<MODE>(a, m.mur[0 + Q], m.mur_lo[0 + Q], v, b);
+    v = {fx ? x.h : v.h, fx ? x.l : v.l};
+    const V<R> y = mur_map<MODE>(b, yh, yl, v, c);
+    v = {fy ? y.h : v.h, fy ? y.l : v.l};
+    const V<R> z = mur_map<MODE>(c, m.mur[9 + Q], m.mur_lo[9 + Q], v, d);
+    return {fz ? z.h : v.h, fz ? z.l : v.l};
 }
 
-template <class R, int MODE>
-__global__ __launch_bounds__(256) void k_faces(Mesh<R> m, long long total) {
-    faces_run<R, MODE, 1>(m, (long long)blockIdx.x * 256, total);
-}
-
-// The same face cells, arranged for one mesh's step.  The rows of the three
-// face planes
+// The rows of the three face planes
 //   X  (Lx, j, k)  0 < j < Ly,   Y0 (i, 0, k), Y1 (i, Ly, k)  i < Lx,   k < Lz
 // take one Mur map of interior cells each:
 //   X  map(cur(Lx-1, j, k), new(Lx-1, j, k), cur(Lx, j, k))
 //   Y0 map(cur(i, 1, k),    new(i, 1, k),    cur(i, 0, k))
 //   Y1 map(cur(i, Ly-1, k), new(i, Ly-1, k), cur(i, Ly, k))
-// (final_value's chain, with after_x and after_y0 reduced to the stage-I
-// value new(), which holds for i < Lx and Ly - 1 > 0).  A wave takes a run
-// of FACE_RUN cells of one row, FACE_LANE_CELLS a lane, and issues all its
-// loads before it stores anything, so one round of memory latency covers
-// them (eight a lane measured no faster than four: the launch is bound by
-// its fixed cost, about 4 us of a 9.6 us launch at 513 x 513 x 257).  The
-// box edges (the rest of face_cell's list, a few thousand cells) go one a
-// thread through final_value, in the last blocks (measured 0.4 us faster
-// per launch than putting them first).  Needs Ly >= 2 for every
-// component.
-constexpr int FACE_LANE_CELLS = 4;                 // cells of a row per lane
-constexpr int FACE_RUN = 64 * FACE_LANE_CELLS;     // cells of a row per wave
-PF_DEV int face_runs(int nz) { return (nz - 1 + FACE_RUN - 1) / FACE_RUN; }
+// (face_value with the one face).  The rows are cut into
+// segments of 64 cells; a wave takes FACE_WAVE_SEGS of them, of as many rows as
+// that is, and issues all its loads before it stores anything, so one round of
+// memory latency covers them.  The launch is bound by that round and its fixed
+// cost, about 4 us (513 x 513 x 257 nodes FP32 7.2 us, 257 x 257 x 129 FP32C
+// 5.4; two segments a wave 8.1 and 5.6, eight 7.6 and 6.4; with rows of up to
+// 256 cells a wave and the edges one a thread through a recursion 8.4 and
+// 9.1).  The box edges, a few thousand cells, go to blocks of their own, the
+// last ones (measured 0.4 us faster per launch than putting them first).
+constexpr int FACE_WAVE_SEGS = 4;
+PF_DEV int face_segs(int nz) { return (nz - 1 + 63) / 64; }
 
 template <int Q>
 PF_DEV int face_rows(int nx, int ny) {
     return Ext<Q>::Ly(ny) - 1 + 2 * Ext<Q>::Lx(nx);
 }
+// Waves of component Q's rows.
+template <int Q>
+PF_DEV int face_waves(int nx, int ny, int nz) {
+    return (face_rows<Q>(nx, ny) * face_segs(nz) + FACE_WAVE_SEGS - 1) / FACE_WAVE_SEGS;
+}
 
+// Wave t of component Q's rows.
 template <int Q, int MODE, class R>
-PF_DEV void face_row_run(const Mesh<R>& m, int r, int run, int lane, R w) {
+PF_DEV void face_row_wave(const Mesh<R>& m, int t, int lane, R w) {
     const int Lx = Ext<Q>::Lx(m.nx), Ly = Ext<Q>::Ly(m.ny), Lz = Ext<Q>::Lz(m.nz);
-    int i, j, ii, ji;  // the face row, the interior row its map reads
-    R mh, ml;          // its Mur coefficient (constant indices: a run-time index
-                       // into the kernel argument would copy it to scratch)
-    if (r < Ly - 1) {
-        i = Lx; j = 1 + r; ii = Lx - 1; ji = j; mh = m.mur[0 + Q]; ml = m.mur_lo[0 + Q];
-    } else if (r < Ly - 1 + Lx) {
-        i = r - (Ly - 1); j = 0; ii = i; ji = 1; mh = m.mur[3 + Q]; ml = m.mur_lo[3 + Q];
-    } else {
-        i = r - (Ly - 1) - Lx; j = Ly; ii = i; ji = Ly - 1; mh = m.mur[6 + Q]; ml = m.mur_lo[6 + Q];
-    }
+    const int ks = face_segs(m.nz), last = face_rows<Q>(m.nx, m.ny) * ks - 1;
     const R* c = Q == 0 ? m.c0 : (Q == 1 ? m.c1 : m.c2);
     const R* n = Q == 0 ? m.n0 : (Q == 1 ? m.n1 : m.n2);
     const lo_t* cl = Q == 0 ? m.cl0 : (Q == 1 ? m.cl1 : m.cl2);
     const lo_t* nl = Q == 0 ? m.nl0 : (Q == 1 ? m.nl1 : m.nl2);
-    const long long fb = at(m, i, j, 0), ib = at(m, ii, ji, 0);
-    V<R> a[FACE_LANE_CELLS], b[FACE_LANE_CELLS], d[FACE_LANE_CELLS];
+    V<R> a[FACE_WAVE_SEGS], b[FACE_WAVE_SEGS], d[FACE_WAVE_SEGS];
+    int i[FACE_WAVE_SEGS], j[FACE_WAVE_SEGS], ii[FACE_WAVE_SEGS], k[FACE_WAVE_SEGS];
+    R mh[FACE_WAVE_SEGS], ml[FACE_WAVE_SEGS];
 #pragma unroll
-    for (int u = 0; u < FACE_LANE_CELLS; u++) {
-        const int k = run * FACE_RUN + u * 64 + lane;
-        const int kk = k < Lz ? k : Lz - 1;  // lanes past the row load its last cell and store nothing
+    for (int u = 0; u < FACE_WAVE_SEGS; u++) {
+        // the face row, the interior row its map reads, its Mur coefficient
+        // (constant indices: a run-time index into the kernel argument would
+        // copy it to scratch)
+        const int g = t * FACE_WAVE_SEGS + u < last ? t * FACE_WAVE_SEGS + u : last;
+        const int r = g / ks;
+        int ji;
+        if (r < Ly - 1) {
+            i[u] = Lx; j[u] = 1 + r; ii[u] = Lx - 1; ji = j[u]; mh[u] = m.mur[0 + Q]; ml[u] = m.mur_lo[0 + Q];
+        } else if (r < Ly - 1 + Lx) {
+            i[u] = r - (Ly - 1); j[u] = 0; ii[u] = i[u]; ji = 1; mh[u] = m.mur[3 + Q]; ml[u] = m.mur_lo[3 + Q];
+        } else {
+            i[u] = r - (Ly - 1) - Lx; j[u] = Ly; ii[u] = i[u]; ji = Ly - 1; mh[u] = m.mur[6 + Q]; ml[u] = m.mur_lo[6 + Q];
+        }
+        const long long fb = at(m, i[u], j[u], 0), ib = at(m, ii[u], ji, 0);
+        k[u] = (g - r * ks) * 64 + lane;
+        const int kk = k[u] < Lz ? k[u] : Lz - 1;  // lanes past the row load its last cell and store nothing
+        if (t * FACE_WAVE_SEGS + u > last) k[u] = Lz;
         a[u].h = c[ib + kk];
         b[u].h = n[ib + kk];
         d[u].h = c[fb + kk];
@@ -471,26 +427,18 @@ PF_DEV void face_row_run(const Mesh<R>& m, int r, int run, int lane, R w) {
         }
     }
 #pragma unroll
-    for (int u = 0; u < FACE_LANE_CELLS; u++) {
-        const int k = run * FACE_RUN + u * 64 + lane;
-        if (k >= Lz) continue;
-        if (Q == 2 && k == 0) {  // the source line uz[0, :, 0] reads as w
-            if (ii == 0) { a[u].h = w; a[u].l = R(0); }
-            if (i == 0) { d[u].h = w; d[u].l = R(0); }
+    for (int u = 0; u < FACE_WAVE_SEGS; u++) {
+        if (k[u] >= Lz) continue;
+        if (Q == 2 && k[u] == 0) {  // the source line uz[0, :, 0] reads as w
+            if (ii[u] == 0) { a[u].h = w; a[u].l = R(0); }
+            if (i[u] == 0) { d[u].h = w; d[u].l = R(0); }
         }
-        put<Q, MODE>(m, i, j, k, mur_map<MODE>(a[u], mh, ml, b[u], d[u]));
+        put<Q, MODE>(m, i[u], j[u], k[u], mur_map<MODE>(a[u], mh[u], ml[u], b[u], d[u]));
     }
 }
 
-template <int Q>
-PF_DEV long long face_edge_base(int nx, int ny, int nz) {
-    const long long Lx = Ext<Q>::Lx(nx), Ly = Ext<Q>::Ly(ny), Lz = Ext<Q>::Lz(nz);
-    return (Ly - 1) * Lz + 2 * Lx * Lz;
-}
-
 // A probe frame recorded by the face launch (probe blocks after the row
-// and edge blocks; blocks = 0: none).  The frame index advances as in
-// k_probe.
+// and edge blocks; blocks = 0: none).
 struct FaceProbe {
     double* ring;
     long long* frame;
@@ -501,12 +449,12 @@ struct FaceProbe {
 // Probe point p of the u_z surface (k = 0) of the level m writes, as a later
 // read would see it.  Points on a u_z face (i = Lx, j = 0 or Ly) are not
 // read: the face blocks of the same launch store them, so the point takes
-// the same chain value (final_value) with its lo part rounded as stored.
+// the same value (face_value) with its lo part rounded as stored.
 template <class R, int MODE>
 PF_DEV double probe_point(const Mesh<R>& m, const FaceProbe& pr, int p, R w) {
     const int i = pr.i0 + pr.si * (p / pr.nj), j = pr.j0 + pr.sj * (p % pr.nj);
     if (i == Ext<2>::Lx(m.nx) || j == 0 || j == Ext<2>::Ly(m.ny)) {
-        const V<R> v = final_value<2, MODE>(m, i, j, 0, w);
+        const V<R> v = face_value<2, MODE>(m, i, j, 0, w);
         double d = (double)v.h;
         if constexpr (MODE == MODE_FP32C) d += (double)lo_decode(v.h, lo_encode(v.h, v.l));
         return d;
@@ -518,33 +466,47 @@ PF_DEV double probe_point(const Mesh<R>& m, const FaceProbe& pr, int p, R w) {
     return d;
 }
 
-// Row block rb of k_faces_rows' grid for view m (four runs, a wave each).
-template <class R, int MODE>
-PF_DEV void face_rows_block(const Mesh<R>& m, int rb, R w) {
-    const int kr = face_runs(m.nz);
+// Row block rb of k_faces_rows' grid (four waves) for the view that view()
+// gives, asked once the component is known: a batch's view is loaded from
+// memory, and only what the component needs of it should be.
+template <class R, int MODE, class View>
+PF_DEV void face_rows_block(int nx, int ny, int nz, const View& view, int rb, R w) {
     const int lane = threadIdx.x % 64;
-    int t = rb * 4 + (int)threadIdx.x / 64;  // this wave's run
-    const int w0 = face_rows<0>(m.nx, m.ny) * kr;
-    if (t < w0) { face_row_run<0, MODE>(m, t / kr, t % kr, lane, w); return; }
+    int t = __builtin_amdgcn_readfirstlane(rb * 4 + (int)threadIdx.x / 64);  // this wave
+    const int w0 = face_waves<0>(nx, ny, nz);
+    if (t < w0) { face_row_wave<0, MODE, R>(view(), t, lane, w); return; }
     t -= w0;
-    const int w1 = face_rows<1>(m.nx, m.ny) * kr;
-    if (t < w1) { face_row_run<1, MODE>(m, t / kr, t % kr, lane, w); return; }
+    const int w1 = face_waves<1>(nx, ny, nz);
+    if (t < w1) { face_row_wave<1, MODE, R>(view(), t, lane, w); return; }
     t -= w1;
-    if (t < face_rows<2>(m.nx, m.ny) * kr) face_row_run<2, MODE>(m, t / kr, t % kr, lane, w);
+    if (t < face_waves<2>(nx, ny, nz)) face_row_wave<2, MODE, R>(view(), t, lane, w);
 }
 
-// Edge block eb (256 box-edge cells, one a thread) for view m.
+// Box-edge cell e of component Q.
+template <int Q, int MODE, class R>
+PF_DEV void face_edge(const Mesh<R>& m, int e, R w) {
+    int i, j, k;
+    face_edge_cell<Q>(m.nx, m.ny, m.nz, e, i, j, k);
+    put<Q, MODE>(m, i, j, k, face_value<Q, MODE>(m, i, j, k, w));
+}
+
+// Edge block eb for view m: FACE_EDGES box-edge cells, spread over its waves.
+// Most edges run along x or y, so each cell reads ten cache lines of its own,
+// and a CU has only so many misses in flight: few cells a block.
+constexpr int FACE_EDGES = 64;
 template <class R, int MODE>
 PF_DEV void face_edges_block(const Mesh<R>& m, int eb, R w) {
-    long long e = (long long)eb * 256 + threadIdx.x;
-    const long long e0 = face_count<0>(m.nx, m.ny, m.nz) - face_edge_base<0>(m.nx, m.ny, m.nz);
-    if (e < e0) { face_write<0, MODE>(m, face_edge_base<0>(m.nx, m.ny, m.nz) + e, w); return; }
+    constexpr int PER = FACE_EDGES / 4;  // a wave's cells
+    const int lane = threadIdx.x % 64;
+    if (lane >= PER) return;
+    int e = eb * FACE_EDGES + (int)threadIdx.x / 64 * PER + lane;
+    const int e0 = face_edges<0>(m.nx, m.ny, m.nz);
+    if (e < e0) { face_edge<0, MODE>(m, e, w); return; }
     e -= e0;
-    const long long e1 = face_count<1>(m.nx, m.ny, m.nz) - face_edge_base<1>(m.nx, m.ny, m.nz);
-    if (e < e1) { face_write<1, MODE>(m, face_edge_base<1>(m.nx, m.ny, m.nz) + e, w); return; }
+    const int e1 = face_edges<1>(m.nx, m.ny, m.nz);
+    if (e < e1) { face_edge<1, MODE>(m, e, w); return; }
     e -= e1;
-    const long long e2 = face_count<2>(m.nx, m.ny, m.nz) - face_edge_base<2>(m.nx, m.ny, m.nz);
-    if (e < e2) face_write<2, MODE>(m, face_edge_base<2>(m.nx, m.ny, m.nz) + e, w);
+    if (e < face_edges<2>(m.nx, m.ny, m.nz)) face_edge<2, MODE>(m, e, w);
 }
 
 template <class R, int MODE>
@@ -571,31 +533,23 @@ __global__ __launch_bounds__(256) void k_faces_rows(Mesh<R> m, int row_blocks, i
         }
         return;
     }
-    if ((int)blockIdx.x < row_blocks) face_rows_block<R, MODE>(m, (int)blockIdx.x, w);
+    if ((int)blockIdx.x < row_blocks)
+        face_rows_block<R, MODE>(m.nx, m.ny, m.nz, [&]() -> const Mesh<R>& { return m; }, (int)blockIdx.x, w);
     else face_edges_block<R, MODE>(m, (int)blockIdx.x - row_blocks, w);
 }
 
-// Blocks of k_faces_rows for an nx x ny x nz mesh: row_blocks (four runs
-// each), then edge_blocks; false when the mesh is too small for it.
-inline bool face_rows_grid(int nx, int ny, int nz, long long& row_blocks, long long& edge_blocks) {
-    if (nx < 3 || ny < 4 || nz < 3) return false;
-    const long long kr = (nz - 1 + FACE_RUN - 1) / FACE_RUN;
-    long long runs = 0, edges = 0;
+// Blocks of k_faces_rows for an nx x ny x nz mesh: row_blocks (four waves
+// each), then edge_blocks.
+inline void face_rows_grid(int nx, int ny, int nz, long long& row_blocks, long long& edge_blocks) {
+    const long long ks = (nz - 1 + 63) / 64;
+    long long waves = 0, edges = 0;
     const long long L[3][3] = {{nx - 2, ny - 1, nz - 1}, {nx - 1, ny - 2, nz - 1}, {nx - 1, ny - 1, nz - 2}};
     for (const auto& e : L) {
-        runs += (e[1] - 1 + 2 * e[0]) * kr;
+        waves += ((e[1] - 1 + 2 * e[0]) * ks + FACE_WAVE_SEGS - 1) / FACE_WAVE_SEGS;
         edges += 2 * (e[2] + 1) + (e[1] - 1) + 2 * e[0];
     }
-    row_blocks = (runs + 3) / 4;
-    edge_blocks = (edges + 255) / 256;
-    return true;
-}
-
-inline long long face_total(int nx, int ny, int nz) {
-    auto cnt = [](long long Lx, long long Ly, long long Lz) {
-        return (Ly - 1) * Lz + 2 * Lx * Lz + 2 * (Lz + 1) + (Ly - 1) + 2 * Lx;
-    };
-    return cnt(nx - 2, ny - 1, nz - 1) + cnt(nx - 1, ny - 2, nz - 1) + cnt(nx - 1, ny - 1, nz - 2);
+    row_blocks = (waves + 3) / 4;
+    edge_blocks = (edges + FACE_EDGES - 1) / FACE_EDGES;
 }
 
 // Stage-I value of one component at a cell: the leapfrog of its current
@@ -668,68 +622,6 @@ __global__ __launch_bounds__(256) void k_sweep_naive(Mesh<R> m) {
     const long long tt = step_index(m);
     if (tt >= m.nsteps) return;
     naive_cell<R, MODE, SPONGE>(m, i, j, k, (R)m.wave[tt]);
-}
-
-// ------------------------------------------------------------ probes ----
-// One probe frame (surface u_z subgrid, hi + lo) into slot `frame % cap` of
-// the ring, after step tt, when (tt + 1) is a multiple of `every`.  Called
-// by all threads of one block; thread 0 advances the frame counter after
-// every read by the block barrier.
-template <class R>
-PF_DEV void probe_record(const R* __restrict__ uz, const lo_t* __restrict__ uzl, long long plane, int pz,
-                         int i0, int si, int ni, int j0, int sj, int nj, double* __restrict__ ring, int cap,
-                         long long* __restrict__ frame, long long tt, int every, long long nsteps) {
-    if (tt >= nsteps || (tt + 1) % every != 0) return;
-    long long f = *frame;
-    double* out = ring + (f % cap) * (long long)ni * nj;
-    for (int p = threadIdx.x; p < ni * nj; p += blockDim.x) {
-        int a = p / nj, b = p % nj;
-        long long id = (long long)(i0 + si * a) * plane + (long long)(j0 + sj * b) * pz;
-        const R h = uz[id];
-        double v = (double)h;
-        if (uzl) v += (double)lo_decode(h, uzl[id]);
-        out[p] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) *frame = f + 1;
-}
-
-// One probe frame of a single mesh, spread over the blocks of the launch:
-// block b gathers points [256 b, 256 b + 256).  Every block reads the frame
-// index, writes its points and counts itself done; the last block to count
-// (after every other block has read the index) advances it and clears the
-// count for the next frame.  No block waits for another.
-template <class R>
-__global__ __launch_bounds__(256) void k_probe(const R* __restrict__ uz, const lo_t* __restrict__ uzl,
-                                               long long plane, int pz, int i0, int si, int ni, int j0, int sj,
-                                               int nj, double* __restrict__ ring, int cap,
-                                               long long* __restrict__ frame, int* __restrict__ done,
-                                               const long long* __restrict__ step_base, long long step_off,
-                                               int every, long long nsteps) {
-    __shared__ int s_last;
-    const long long tt = (step_base ? *step_base : 0) + step_off;  // step just completed
-    if (tt >= nsteps || (tt + 1) % every != 0) return;             // the same for every block
-    const long long f = *frame;
-    double* out = ring + (f % cap) * (long long)ni * nj;
-    const int p = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (p < ni * nj) {
-        const int a = p / nj, b = p % nj;
-        const long long id = (long long)(i0 + si * a) * plane + (long long)(j0 + sj * b) * pz;
-        const R h = uz[id];
-        double v = (double)h;
-        if (uzl) v += (double)lo_decode(h, uzl[id]);
-        out[p] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        s_last = atomicAdd(done, 1) == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (s_last && threadIdx.x == 0) {
-        *frame = f + 1;
-        *done = 0;
-    }
 }
 
 // Tiny kernel: advance a device step counter after a captured chunk.
