@@ -181,7 +181,8 @@ PF_DEV R div3_uz_surface(R d1, R g1, R d2, R g2, R t3k1, R t3k0, R fz0) {
 }
 
 // ---- leapfrog ---------------------------------------------------------------
-// u_new = 2 u - u_old + coef * div (base_solver.py:441-443).  With a damping
+// u_new = 2 u - u_old + coef * div (base_solver.py:441-443); 2 u is exact, so
+// the difference takes one fused operation.  With a damping
 // term s > 0 (sponge extension): ((2u - (1-s) u_old) + coef*div) / (1+s);
 // in FP32 the division is a product with the hardware reciprocal of 1+s
 // (v_rcp_f32, within 1 ulp; one per node, shared by its three components:
@@ -195,14 +196,14 @@ PF_DEV R leap(R u, R uo, R coef, R dv, R s) {
         if constexpr (SPONGE) {
             // off the absorbing layer s = 0: (1 - 0) u_old = u_old and
             // x / (1 + 0) = x exactly, so the division is skipped there
-            R r = 2 * u - (1 - s) * uo + coef * dv;
+            R r = mad(R(2), u, -((1 - s) * uo)) + coef * dv;
             if (s != R(0)) r = r / (1 + s);
             return r;
         }
-        else return 2 * u - uo + coef * dv;
+        else return mad(R(2), u, -uo) + coef * dv;
     } else {
-        if constexpr (SPONGE) return mad(coef, dv, 2 * u - (1 - s) * uo) * __builtin_amdgcn_rcpf(1 + s);
-        else return mad(coef, dv, 2 * u - uo);
+        if constexpr (SPONGE) return mad(coef, dv, mad(R(2), u, -((1 - s) * uo))) * __builtin_amdgcn_rcpf(1 + s);
+        else return mad(coef, dv, mad(R(2), u, -uo));
     }
 }
 
@@ -211,14 +212,17 @@ PF_DEV R leap(R u, R uo, R coef, R dv, R s) {
 // so lo is kept as a signed 16-bit multiple of 2^-16 ulp(hi) (ulp(hi) =
 // 2^(e-24) for hi = m 2^e, 0.5 <= |m| < 1): hi + lo carries 24 + 16
 // significant bits in 6 bytes instead of 8.  Both functions are exact
-// scalings (ldexp) around one round-to-nearest; hi = 0 has lo = 0.
+// scalings (ldexp) around one round-to-nearest; hi = 0 has lo = 0.  The sum
+// with 1.5 x 2^23 rounds to an integer, ties to even, and leaves it in its low
+// bits (one operation for the rounding and the conversion).  This, the sums
+// with 2 u and the short last sum of the damped update took 385 x 371 x 193 nodes
+// FP32C from 451 to 431 us a step (62 % of the issue slots are VALU work there).
 typedef int16_t lo_t;
 
 PF_DEV lo_t lo_encode(float hi, float lo) {
     const int e = __builtin_amdgcn_frexp_expf(hi);
-    float q = __builtin_rintf(__builtin_amdgcn_ldexpf(lo, 40 - e));
-    q = fminf(fmaxf(q, -32767.0f), 32767.0f);
-    return (lo_t)(int)q;
+    const float q = __builtin_amdgcn_fmed3f(__builtin_amdgcn_ldexpf(lo, 40 - e), -32767.0f, 32767.0f);
+    return (lo_t)__float_as_int(q + 12582912.0f);
 }
 PF_DEV float lo_decode(float hi, lo_t q) {
     return __builtin_amdgcn_ldexpf((float)q, __builtin_amdgcn_frexp_expf(hi) - 40);
@@ -234,6 +238,17 @@ PF_DEV void two_sum(float a, float b, float& s, float& e) {
     float bb = s - a;
     e = (a - (s - bb)) + (b - bb);
 }
+// two_sum(2 a, b): 2 a is exact, so it needs no operation of its own.
+PF_DEV void two_sum_2a(float a, float b, float& s, float& e) {
+    s = mad(2.0f, a, b);
+    float bb = mad(-2.0f, a, s);
+    e = mad(2.0f, a, -(s - bb)) + (b - bb);
+}
+// two_sum for |a| >= |b| or a = b = 0 (Dekker): the same s and e.
+PF_DEV void fast_two_sum(float a, float b, float& s, float& e) {
+    s = a + b;
+    e = b - (s - a);
+}
 
 // U_new = 2 U - U_old + f (+ damping), with U = hi + lo.  The increment f is
 // an ordinary FP32 value; what is compensated is the accumulation of the
@@ -243,8 +258,8 @@ template <bool SPONGE>
 PF_DEV void leap_comp(float hi, float lo, float ohi, float olo, float f, float s, float& nhi, float& nlo) {
     if constexpr (!SPONGE) {
         float a, e;
-        two_sum(2.0f * hi, -ohi, a, e);
-        float low = ((2.0f * lo - olo) + e) + f;
+        two_sum_2a(hi, -ohi, a, e);
+        float low = (mad(2.0f, lo, -olo) + e) + f;
         two_sum(a, low, nhi, nlo);
     } else {
         float q = 1.0f - s;
@@ -252,14 +267,15 @@ PF_DEV void leap_comp(float hi, float lo, float ohi, float olo, float f, float s
         float pe = mad(q, ohi, -p);
         float plow = mad(q, olo, pe);
         float a, e;
-        two_sum(2.0f * hi, -p, a, e);
-        float low = ((2.0f * lo - plow) + e) + f;
+        two_sum_2a(hi, -p, a, e);
+        float low = (mad(2.0f, lo, -plow) + e) + f;
         float nh, nl;
         two_sum(a, low, nh, nl);
         float r = __builtin_amdgcn_rcpf(1.0f + s);  // as in leap()
         float h2 = nh * r;
         float l2 = mad(nh, r, -h2) + nl * r;
-        two_sum(h2, l2, nhi, nlo);
+        // |nl| <= ulp(nh) / 2 and r > 1 / 2: |l2| < 2 ulp(h2) <= |h2|
+        fast_two_sum(h2, l2, nhi, nlo);
     }
 }
 
