@@ -650,12 +650,7 @@ static int launch_faces_probe_t(const pf_ctx* c, const Mesh<R>& m, hipStream_t s
 template <class R, int MODE>
 static Mesh<R> sweep_view(const pf_ctx* c, int cur, int old, int nxt) {
     Mesh<R> m = make_view<R>(c, cur, old, nxt);
-    if constexpr (MODE == MODE_FP64P) {
-        m.fx = m.rfx; m.fy = m.rfy; m.fz = m.rfz;
-        m.sx = m.rsx; m.sy = m.rsy; m.sz = m.rsz;
-        m.fx0 = m.rfx0; m.fy0 = m.rfy0; m.fz0 = m.rfz0;
-        m.sx0 = m.rsx0; m.sy0 = m.rsy0; m.sz0 = m.rsz0;
-    }
+    take_spacings<MODE>(m);
     return m;
 }
 
@@ -670,7 +665,7 @@ static int step_once_t(pf_ctx* c, hipStream_t s, const long long* base, long lon
     if ((rc = launch_sweep_t<R, MODE>(c, m, s))) return rc;
     if (ev) HIPCHK(hipEventRecord(ev[1], s));
     // the faces read no spacings: the FP64 face kernels serve all FP64 modes
-    if ((rc = launch_faces_probe_t<R, MODE == MODE_FP64P || MODE == MODE_FP64Q ? MODE_FP64 : MODE>(c, m, s))) return rc;
+    if ((rc = launch_faces_probe_t<R, face_mode(MODE)>(c, m, s))) return rc;
     const int t = c->cur;
     c->cur = c->old;
     c->old = t;

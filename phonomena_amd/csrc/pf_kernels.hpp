@@ -94,6 +94,18 @@ PF_DEV long long at(const Mesh<R>& m, int i, int j, int k) {
     return (long long)i * m.plane + (long long)j * m.pz + k;
 }
 
+// The spacings a sweep of MODE reads: with MODE_FP64P the tables and first
+// spacings are the exact reciprocals.
+template <int MODE, class R>
+inline void take_spacings(Mesh<R>& m) {
+    if constexpr (MODE == MODE_FP64P) {
+        m.fx = m.rfx; m.fy = m.rfy; m.fz = m.rfz;
+        m.sx = m.rsx; m.sy = m.rsy; m.sz = m.rsz;
+        m.fx0 = m.rfx0; m.fy0 = m.rfy0; m.fz0 = m.rfz0;
+        m.sx0 = m.rsx0; m.sy0 = m.rsy0; m.sz0 = m.rsz0;
+    }
+}
+
 template <class R>
 PF_DEV long long step_index(const Mesh<R>& m) {
     return (m.step_base ? *m.step_base : 0) + m.step_off;
@@ -436,6 +448,9 @@ PF_DEV void face_row_wave(const Mesh<R>& m, int t, int lane, R w) {
         put<Q, MODE>(m, i[u], j[u], k[u], mur_map<MODE>(a[u], mh[u], ml[u], b[u], d[u]));
     }
 }
+
+// The faces read no spacings: one kernel serves all FP64 modes.
+constexpr int face_mode(int mode) { return mode == MODE_FP64P || mode == MODE_FP64Q ? MODE_FP64 : mode; }
 
 // A probe frame recorded by the face launch (probe blocks after the row
 // and edge blocks; blocks = 0: none).
