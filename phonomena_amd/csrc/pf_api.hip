@@ -1205,7 +1205,7 @@ extern "C" int pf_energy(pf_ctx* c, double* out) {
     if (!c || !out) return fail(PF_ERR_ARG, "NULL argument");
     hipStream_t s = c->batch ? c->batch_stream : c->stream;
     // about 8 blocks per CU, 4 to ENERGY_XCHUNK planes each
-    const long long per = (c->plane + 255) / 256;
+    const long long per = (c->plane + ENERGY_CELLS - 1) / ENERGY_CELLS;
     long long want = (2048 + per - 1) / per;
     if (want > (c->nx + 3) / 4) want = (c->nx + 3) / 4;
     int xc = (int)((c->nx + want - 1) / want);

@@ -5,14 +5,15 @@
 //
 // A thread takes one (y, z) cell of the planes of an x chunk.  It keeps the
 // plane's and the next plane's own values in registers; the neighbours along
-// y and z are loads that hit the lines its wave's and the next row's own
-// values bring in, so a level is read from HBM once.  Strains are formed once
-// per level and site with reciprocal spacings (1 ulp from a quotient; the
-// FP64 divisions they replace, thirty a node, were most of the kernel's
-// time), stresses from the newest level's.  Bound: instructions (the decoded
-// neighbours in FP32C, FP64 arithmetic in the others), then the two levels'
-// bytes.  A call on 257 x 257 x 129 nodes takes 164 us in FP32C, 95 in FP32,
-// 150 in FP64, against 680, 621 and 453 with levels widened to FP64 arrays by
+// z are lane shifts (a wave's outer lanes repeat its neighbours' cells), those
+// along y loads that hit the lines the next row's own values bring in, so a
+// level is read from HBM once.  Strains are formed once per level and site
+// with reciprocal spacings (1 ulp from a quotient; the FP64 divisions they
+// replace, thirty a node, were most of the kernel's time), stresses from the
+// newest level's.  Bound: instructions and the waves in flight (122 VGPRs, 146
+// in FP32C).  A call on 257 x 257 x 129 nodes takes 128 us in FP32C, 83 in
+// FP32, 130 in FP64 (166, 95 and 150 with the z neighbours loaded and decoded
+// again), against 680, 621 and 453 with levels widened to FP64 arrays by
 // six launches first and a grid-stride kernel with 64-bit index divisions and
 // quotients per node; 20 us on small meshes (81 and 40).  The relative error
 // against a 64-bit restatement is the same (2e-16 to 8e-16 in FP64).
@@ -20,7 +21,7 @@
 // Per-thread sums, a wavefront/LDS tree per block, then one block adds the
 // block partials in a fixed order, so the result is deterministic.
 #pragma once
-#include "pf_kernels.hpp"
+#include "pf_tiled.hpp"
 
 namespace pf {
 
@@ -32,7 +33,7 @@ struct EnergyArgs {
     double dt;
     const double* w_prev;      // source of the step that produced the newest level (null: none)
     int xchunk;                // planes per block
-    unsigned per;              // blocks per chunk: block b takes cells 256 (b % per) ... of chunk b / per
+    unsigned per;              // blocks per chunk: block b takes cells ENERGY_CELLS (b % per) ... of chunk b / per
 };
 
 PF_DEV double warp_sum(double v) {
@@ -41,6 +42,7 @@ PF_DEV double warp_sum(double v) {
 }
 
 constexpr int ENERGY_XCHUNK = 32;  // most planes per block
+constexpr int ENERGY_CELLS = 4 * 62;  // cells per block: a wave's outer lanes are its neighbours' cells
 
 // One level's value of a component at cell a of its array.
 template <bool COMP, class R>
@@ -77,8 +79,14 @@ __global__ __launch_bounds__(256) void k_energy_partial(Mesh<R> m, EnergyArgs ea
     }
     __syncthreads();
     double ke = 0.0, se = 0.0;
-    const long long plane = m.plane, t = (long long)(blockIdx.x % ea.per) * 256 + threadIdx.x;
-    if (t < plane) {
+    const long long plane = m.plane;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // cells before the plane's first and past its last take those (and, as
+    // every outer lane, add nothing)
+    long long t = (long long)(blockIdx.x % ea.per) * ENERGY_CELLS + wv * 62 + lane - 1;
+    const bool own = lane >= 1 && lane <= 62 && t < plane;
+    t = t < 0 ? 0 : (t < plane ? t : plane - 1);
+    {
         const int j = (int)(t / m.pz), k = (int)(t % m.pz);
         const bool ks = k >= 1, kf = k <= m.nz - 2, jn = j >= 1 && j <= m.ny - 2, jf = j <= m.ny - 2;
         // k = 0 takes the first spacings, in the reference's order (as the
@@ -90,9 +98,10 @@ __global__ __launch_bounds__(256) void k_energy_partial(Mesh<R> m, EnergyArgs ea
         const double rsx0 = 1.0 / ea.s0[0], rdt = 1.0 / ea.dt;
         const double h41 = ks ? rfz : rfy0, h42 = ks ? rfy : rfz0, h51 = ks ? rfz : rfx0, h61 = ks ? rfy : rfx0;
         const double wp = ea.w_prev && k == 0 && i0 == 0 ? *ea.w_prev : 0.0;
-        // neighbours inside the plane (cells without one read themselves:
-        // their terms are left out)
-        const long long jp = jf ? m.pz : 0, jm = j >= 1 ? m.pz : 0, kp = k <= m.nz - 2 ? 1 : 0, km = ks ? 1 : 0;
+        // neighbours inside the plane: along y cells without one read
+        // themselves, along z the lanes beside take the next row's; their
+        // terms are left out
+        const long long jp = jf ? m.pz : 0, jm = j >= 1 ? m.pz : 0, kp = k <= m.nz - 2 ? 1 : 0;
         const long long kq = ks ? kp : 0;
         long long a = (long long)i0 * plane + t;
         // own values: [level][component], planes i and i+1, ux of plane i-1
@@ -130,12 +139,12 @@ __global__ __launch_bounds__(256) void k_energy_partial(Mesh<R> m, EnergyArgs ea
                 const bool sub = l && i == 0 && k == 0 && ea.w_prev;
                 const double z = sub ? wp : u[l][2];
                 const double zj = sub ? wp : energy_at<COMP>(h2, l2, a + jp);
-                const double zm = ks ? energy_at<COMP>(h2, l2, a - km) : 0.0;
+                const double zb = below0(u[l][2]), zm = ks ? zb : 0.0;
                 s[l].e1 = (u[l][0] - uxm[l]) * rsx;
                 s[l].e2 = (u[l][1] - energy_at<COMP>(h1, l1, a - jm)) * ry;
                 s[l].e3 = (z - zm) * rz;
-                s[l].g4 = (energy_at<COMP>(h1, l1, a + kp) - u[l][1]) * h41 + (zj - z) * h42;
-                s[l].g5 = (energy_at<COMP>(h0, l0, a + kp) - u[l][0]) * h51 + (un[l][2] - z) * h52;
+                s[l].g4 = (above0(u[l][1]) - u[l][1]) * h41 + (zj - z) * h42;
+                s[l].g5 = (above0(u[l][0]) - u[l][0]) * h51 + (un[l][2] - z) * h52;
                 s[l].g6 = (energy_at<COMP>(h0, l0, a + jp) - u[l][0]) * h61 + (un[l][1] - u[l][1]) * h52;
             }
             if (is && jn && kf) {
@@ -172,9 +181,8 @@ __global__ __launch_bounds__(256) void k_energy_partial(Mesh<R> m, EnergyArgs ea
             id_k = in_k;
         }
     }
-    ke = warp_sum(ke);
-    se = warp_sum(se);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    ke = warp_sum(own ? ke : 0.0);
+    se = warp_sum(own ? se : 0.0);
     if (lane == 0) { red[0][wv] = ke; red[1][wv] = se; }
     __syncthreads();
     if (threadIdx.x == 0) {
