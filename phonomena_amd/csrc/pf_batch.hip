@@ -246,7 +246,8 @@ void free_tables(pf_batch* b) {
 // Default rows x lanes of a batch (the autotuner refines them): 16 x 32, 8 x
 // 32 in FP64.  Members are a few times 30 nodes deep, so 62-lane tiles leave
 // lanes idle, and 32 rows make few work items of a small batch.  Measured,
-// microseconds a step at each shape's best chunk, 16 x 32 / 16 x 64 / 8 x 64 /
+// microseconds a step at each shape's best chunk (with the earlier face and
+// probe launches, 10 to 16 us more), 16 x 32 / 16 x 64 / 8 x 64 /
 // 32 x 32 / 8 x 32: 16 members of 14.2 M nodes FP32C 312 / 315 / 312 / 315 /
 // 335; 10 of 2.8 M 88 / 92 / 95 / 91 / 92; 5 of 1.4 M 64 / 61 / 67 / 62 / 67.
 // From 2^25 nodes on, where every shape keeps the chip full, 16 x 64 (FP32 and
