@@ -970,6 +970,8 @@ static hipError_t unpack(pf_ctx* c, int lvl, int q, long long first, long long c
 
 static int ensure_scratch(pf_ctx* c, size_t bytes) {
     if (c->scratch_bytes >= bytes) return PF_OK;
+    const OnDevice on(c->dev);
+    HIPCHK(on.error);
     if (c->scratch) HIPCHK(hipFree(c->scratch));
     c->scratch = nullptr;
     c->scratch_bytes = 0;

@@ -132,6 +132,27 @@ inline unsigned long long level_bytes(long long cells, int precision) {
 }
 
 int fail(int code, const char* fmt, ...);
+
+// Device dev current for a scope: a caller may have another one current when
+// it uses a context, and what is made for the context (memory, streams,
+// events) has to be on the context's device.
+struct OnDevice {
+    hipError_t error;
+    int was = -1;
+    explicit OnDevice(int dev) {
+        int cur = -1;
+        error = hipGetDevice(&cur);
+        if (error != hipSuccess || cur == dev) return;
+        error = hipSetDevice(dev);
+        if (error == hipSuccess) was = cur;
+    }
+    ~OnDevice() {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+};
+
 int ctx_init(pf_ctx* c, const pf_desc* d);
 void ctx_free(pf_ctx* c);
 // View of a step from level `cur` (n) and `old` (n-1) into level `out`.

@@ -75,7 +75,7 @@ hipError_t on_lanes(int dev, size_t chunks, F work) {
 
 // The device with the lanes that a transfer of `bytes` works, made on first
 // use, for as long as `lock` is held; null when they are taken or cannot be
-// made.
+// made.  Device dev is current.
 Device* lanes_of(int dev, size_t bytes, std::unique_lock<std::mutex>& lock) {
     if (dev < 0 || dev >= MAX_DEVICES) return nullptr;
     Device& d = g_dev[dev];
@@ -114,6 +114,8 @@ hipError_t copy8(hipStream_t s, void* dst, const void* src, size_t bytes) {
 }  // namespace
 
 int stage_out(int dev, hipStream_t after, void* host, size_t bytes, const StageFill& fill, bool* taken) {
+    const OnDevice on(dev);
+    HIPCHK(on.error);
     std::unique_lock<std::mutex> lock;
     Device* const st = lanes_of(dev, bytes, lock);
     *taken = st != nullptr;
@@ -149,6 +151,8 @@ int stage_out(int dev, hipStream_t after, void* host, size_t bytes, const StageF
 }
 
 int stage_in(int dev, hipStream_t after, const void* host, size_t bytes, const StageDrain& drain, bool* taken) {
+    const OnDevice on(dev);
+    HIPCHK(on.error);
     std::unique_lock<std::mutex> lock;
     Device* const st = lanes_of(dev, bytes, lock);
     *taken = st != nullptr;

@@ -1,0 +1,72 @@
+"""The library's host code over a stand-in HIP runtime (host_runtime.cpp: two
+devices, kernels that do nothing), without a GPU: which device its objects
+are made on, what it allocates and when, what it launches.  Every case runs
+in a process of its own, whose HIP calls all come to the stand-in."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, sys
+sys.path[:0] = [%r, %r]
+hip = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
+hip.host_count.restype = ctypes.c_longlong
+hip.host_launch.restype = ctypes.c_char_p
+import numpy as np
+from helpers import spec_from, uniform_crystal
+from phonomena_amd import fdtd
+
+def count(what):
+    return hip.host_count(what.encode())
+
+def launches():
+    return [hip.host_launch(i).decode() for i in range(hip.host_launches())]
+
+def device():
+    d = ctypes.c_int()
+    hip.hipGetDevice(ctypes.byref(d))
+    return d.value
+
+def context(cells, precision="fp64", kernel="auto", tune=False, steps=40, spacing=1.0, **kw):
+    x, y, z, ids, rows, dt, wave = uniform_crystal(cells, spacing, steps=steps)
+    return fdtd.Context(spec_from(x, y, z, ids, rows, dt, wave, **kw), precision=precision, kernel=kernel, tune=tune)
+"""
+
+
+@pytest.fixture(scope="session")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "host_runtime.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-o", so, os.path.join(HERE, "host_runtime.cpp")],
+                   check=True)
+    return so
+
+
+def run(runtime, body):
+    r = subprocess.run([sys.executable, "-c", PRELUDE % (ROOT, HERE, runtime) + body], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("current", [0, 1])
+@pytest.mark.parametrize("pinned", [True, False])  # without pinned memory a transfer goes through device scratch
+def test_transfers_of_a_context_stay_on_its_device(runtime, current, pinned):
+    run(runtime, """
+hip.hipSetDevice(1)
+c = context((70, 40, 40), probe=(0, 1, 70, 0, 1, 40), every=1)
+hip.hipSetDevice(%d)
+hip.host_fail_host_malloc(%d)
+c.step(2)
+for f in ("ux", "uy_old"):
+    c.get(f)
+    c.set(f, np.zeros(c._shapes[f[:2]]))
+c.probes()
+assert device() == %d
+for what in ("malloc", "host_malloc", "stream", "event"):
+    assert count(what + "@0") == 0, what
+assert (count("host_malloc@1") > 0) == %s
+""" % (current, not pinned, current, pinned))
