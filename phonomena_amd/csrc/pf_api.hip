@@ -306,6 +306,19 @@ static void block_plan(pf_ctx* c) {
             c->block_steps = r;
         }
     }
+    for (int r = 1; r <= c->block_steps; r++) {
+        hipError_t e = hipSuccess;
+        if (c->precision == PF_FP64 && c->recip)
+            e = c->sponge ? allow_block_k<double, MODE_FP64P, true>(c->block[r])
+                          : allow_block_k<double, MODE_FP64P, false>(c->block[r]);
+        else if (c->precision == PF_FP64)
+            e = c->sponge ? allow_block_k<double, MODE_FP64, true>(c->block[r])
+                          : allow_block_k<double, MODE_FP64, false>(c->block[r]);
+        if (e != hipSuccess) {  // no room for such blocks here: march
+            (void)hipGetLastError();
+            c->block_steps = 0;
+        }
+    }
     if (c->block_steps) c->shape_open = false;
 }
 

@@ -419,9 +419,6 @@ int launch_block_m(const Mesh<R>& m, const BlockMap& bm, R* const* p, lo_t* cons
                    hipStream_t s) {
     const auto kernel = k_block_steps<R, MODE, SPONGE, MOST>;
     const size_t lds = block_lds<R, MODE>(bm.threads);
-    static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)block_lds<R, MODE>(MOST));
-    if (room != hipSuccess) return fail(PF_ERR_HIP, "block steps: %s", hipGetErrorString(room));
     hipLaunchKernelGGL(kernel, dim3((unsigned)(bm.ntx * bm.nty * bm.ntz)), dim3((unsigned)bm.threads), lds, s, m, p[0],
                        p[1], p[2], pl[0], pl[1], pl[2], bm, bm.steps, pr);
     HIPCHK(hipGetLastError());
@@ -435,6 +432,18 @@ int launch_block_k(const Mesh<R>& m, const BlockMap& bm, R* const* p, lo_t* cons
                    hipStream_t s) {
     return bm.threads <= 512 ? launch_block_m<R, MODE, SPONGE, 512>(m, bm, p, pl, pr, s)
                              : launch_block_m<R, MODE, SPONGE, BLOCK_MAX_NODES>(m, bm, p, pl, pr, s);
+}
+
+// Allows the kernel that takes blocks of bm its LDS on the current device (only
+// the largest blocks in FP64 need more than every kernel may have).
+template <class R, int MODE, bool SPONGE>
+hipError_t allow_block_k(const BlockMap& bm) {
+    const size_t lds = block_lds<R, MODE>(bm.threads);
+    if (lds <= 64u << 10) return hipSuccess;
+    const void* kernel = bm.threads <= 512 ? (const void*)k_block_steps<R, MODE, SPONGE, 512>
+                                           : (const void*)k_block_steps<R, MODE, SPONGE, BLOCK_MAX_NODES>;
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)block_lds<R, MODE>(BLOCK_MAX_NODES));
 }
 
 }  // namespace pf

@@ -21,6 +21,7 @@ struct Event { int dev; int at; };
 
 static std::mutex g_lock;
 static thread_local int t_dev = 0;
+static thread_local hipError_t t_error = 0;  // of a launch
 static std::map<const void*, std::string> g_names;
 static std::map<std::pair<const void*, int>, int> g_lds;  // (kernel, device) -> dynamic LDS allowed
 static std::map<void*, int> g_owner;                       // memory -> device
@@ -61,7 +62,11 @@ hipError_t hipGetDevice(int* d) { *d = t_dev; return 0; }
 hipError_t hipDeviceGetAttribute(int* v, int, int) { *v = 256; return 0; }
 hipError_t hipGetDevicePropertiesR0600(void*, int) { return 101; }
 const char* hipGetErrorString(hipError_t) { return "refused by the stand-in runtime"; }
-hipError_t hipGetLastError() { return 0; }
+hipError_t hipGetLastError() {
+    const hipError_t e = t_error;
+    t_error = 0;
+    return e;
+}
 
 // ---- memory ----
 static hipError_t take(void** p, size_t n, const char* what) {
@@ -138,10 +143,11 @@ hipError_t hipFuncSetAttribute(const void* f, int, int v) {
 hipError_t hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t lds, Stream* s) {
     const int dev = dev_of(s);
     count("launch", dev);
+    if (lds > 65536) count("large_lds", dev);
     std::lock_guard<std::mutex> l(g_lock);
     g_launches.push_back(g_names[f]);
     auto room = g_lds.find({f, dev});
-    if ((long long)lds > (room == g_lds.end() ? 65536 : room->second)) return 1;
+    if ((long long)lds > (room == g_lds.end() ? 65536 : room->second)) return t_error = 1;
     return 0;
 }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { *n = 2; return 0; }

@@ -70,3 +70,15 @@ for what in ("malloc", "host_malloc", "stream", "event"):
     assert count(what + "@0") == 0, what
 assert (count("host_malloc@1") > 0) == %s
 """ % (current, not pinned, current, pinned))
+
+
+def test_the_largest_blocks_get_their_lds_on_every_device(runtime):
+    run(runtime, """
+for dev in (0, 1):
+    hip.hipSetDevice(dev)
+    for cells in ((49, 94, 23), (74, 98, 17)):
+        c = context(cells, tune=True, spacing=0.3)
+        c.step(4)
+        c.close()
+    assert count("large_lds@%d" % dev) > 0
+""")
