@@ -141,7 +141,7 @@ typedef struct pf_desc {
 } pf_desc;
 
 /* Frees the pinned staging memory that transfers keep between calls (at most
-   8 MiB a device; all but 1 MiB of it also goes with a device's last
+   32 MiB a device; what is above 8 MiB also goes with a device's last
    context). */
 int pf_trim(void);
 

@@ -1,5 +1,5 @@
-// Staged transfers (pf_stage.hpp): the lanes of each device and the host
-// threads that work them.
+// Staged transfers (pf_stage.hpp): the pinned memory of each device and the
+// host threads that work through it.
 #include "pf_stage.hpp"
 
 #include <cstring>
@@ -14,43 +14,53 @@ namespace {
 
 constexpr int MAX_DEVICES = 64;
 
-struct Lane {
-    hipStream_t stream = nullptr;
-    char* chunk[2] = {};
-    hipEvent_t done[2] = {};
-};
+constexpr int SLOTS = 2 * STAGE_LANES;
+
 struct Device {
-    std::mutex use;              // held for a transfer
-    Lane lane[STAGE_LANES];      // those made so far, from the front
-    hipEvent_t ready = nullptr;
+    std::mutex use;  // held for a transfer
+    char* pinned = nullptr;
+    size_t room = 0;
+    hipEvent_t done[SLOTS] = {};  // a slot's chunk has been written or read
     std::mutex count;
-    int users = 0;               // contexts
+    int users = 0;  // contexts
 };
 Device g_dev[MAX_DEVICES];
 
-void destroy(Lane& l) {
-    for (int k = 0; k < 2; k++) {
-        if (l.chunk[k]) (void)hipHostFree(l.chunk[k]);
-        if (l.done[k]) (void)hipEventDestroy(l.done[k]);
-    }
-    if (l.stream) (void)hipStreamDestroy(l.stream);
-    l = Lane();
+void give_back(Device& d) {
+    if (d.pinned) (void)hipHostFree(d.pinned);
+    d.pinned = nullptr;
+    d.room = 0;
 }
 
-hipError_t create(Lane& l) {
-    hipError_t e = hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking);
-    for (int k = 0; k < 2; k++) {
-        if (e == hipSuccess) e = hipHostMalloc((void**)&l.chunk[k], STAGE_CHUNK, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&l.done[k], hipEventDisableTiming);
-    }
+// At least `bytes` of pinned memory, and the events.
+hipError_t reserve(Device& d, size_t bytes) {
+    hipError_t e = hipSuccess;
+    for (hipEvent_t& v : d.done)
+        if (!v && e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+    if (e != hipSuccess || d.room >= bytes) return e;
+    give_back(d);
+    e = hipHostMalloc((void**)&d.pinned, bytes, hipHostMallocDefault);
+    if (e == hipSuccess) d.room = bytes;
+    else d.pinned = nullptr;
     return e;
 }
 
-// Runs work(lane) on as many lanes as the transfer has chunks for, the
-// caller's thread among them; lanes whose thread cannot start run here.
+// A transfer's chunks: chunk c belongs to lane c % lanes, whose chunks take
+// its two slots in turn.
+struct Ring {
+    Device* d;
+    size_t bytes, chunk, chunks;
+    int lanes;
+    size_t len(size_t c) const { return c + 1 < chunks ? chunk : bytes - c * chunk; }
+    int slot(size_t c) const { return (int)(c % (size_t)(2 * lanes)); }
+    char* at(size_t c) const { return d->pinned + (size_t)slot(c) * chunk; }
+    hipEvent_t done(size_t c) const { return d->done[slot(c)]; }
+};
+
+// Runs work(lane) for every lane, lane 0 on the caller's thread; lanes whose
+// thread cannot start run here.
 template <class F>
-hipError_t on_lanes(int dev, size_t chunks, F work) {
-    const int lanes = (int)(chunks < (size_t)STAGE_LANES ? chunks : STAGE_LANES);
+hipError_t on_lanes(int dev, int lanes, F work) {
     hipError_t err[STAGE_LANES];
     for (auto& e : err) e = hipSuccess;
     std::thread t[STAGE_LANES];
@@ -58,45 +68,35 @@ hipError_t on_lanes(int dev, size_t chunks, F work) {
         try {
             t[w] = std::thread([&, w] {
                 err[w] = hipSetDevice(dev);
-                if (err[w] == hipSuccess) err[w] = work(w, lanes);
+                if (err[w] == hipSuccess) err[w] = work(w);
             });
         } catch (const std::system_error&) {
         }
     }
-    err[0] = work(0, lanes);
+    err[0] = work(0);
     for (int w = 1; w < lanes; w++) {
         if (t[w].joinable()) t[w].join();
-        else err[w] = work(w, lanes);
+        else err[w] = work(w);
     }
     for (int w = 0; w < lanes; w++)
         if (err[w] != hipSuccess) return err[w];
     return hipSuccess;
 }
 
-// The device with the lanes that a transfer of `bytes` works, made on first
-// use, for as long as `lock` is held; null when they are taken or cannot be
-// made.  Device dev is current.
-Device* lanes_of(int dev, size_t bytes, std::unique_lock<std::mutex>& lock) {
-    if (dev < 0 || dev >= MAX_DEVICES) return nullptr;
+// The ring for a transfer of `bytes` in chunks of `chunk`, for as long as
+// `lock` is held; d = null when the device's is taken or cannot be made.
+// Device dev is current.
+Ring ring_of(int dev, size_t bytes, size_t chunk, std::unique_lock<std::mutex>& lock) {
+    Ring r = {nullptr, bytes, chunk, (bytes + chunk - 1) / chunk, 1};
+    if (r.chunks > 1) r.lanes = (int)(r.chunks < (size_t)STAGE_LANES ? r.chunks : STAGE_LANES);
+    if (dev < 0 || dev >= MAX_DEVICES) return r;
     Device& d = g_dev[dev];
     lock = std::unique_lock<std::mutex>(d.use, std::try_to_lock);
-    if (!lock.owns_lock()) return nullptr;
-    hipError_t e = d.ready ? hipSuccess : hipEventCreateWithFlags(&d.ready, hipEventDisableTiming);
-    for (int w = 0; w < STAGE_LANES && (size_t)w * STAGE_CHUNK < bytes && e == hipSuccess; w++)
-        if (!d.lane[w].stream && (e = create(d.lane[w])) != hipSuccess) destroy(d.lane[w]);
-    if (e == hipSuccess) return &d;
-    (void)hipGetLastError();
-    return nullptr;
-}
-
-// Frees the lanes from `first` on.
-void give_back(Device& d, int first) {
-    std::lock_guard<std::mutex> lock(d.use);
-    for (int w = first; w < STAGE_LANES; w++) destroy(d.lane[w]);
-    if (first == 0 && d.ready) {
-        (void)hipEventDestroy(d.ready);
-        d.ready = nullptr;
-    }
+    if (!lock.owns_lock()) return r;
+    const size_t slots = r.chunks < SLOTS ? r.chunks : SLOTS;
+    if (reserve(d, slots * chunk) == hipSuccess) r.d = &d;
+    else (void)hipGetLastError();
+    return r;
 }
 
 // A copy on the device's side of PCIe: n8 eight-byte words.  A kernel moves a
@@ -116,72 +116,61 @@ hipError_t copy8(hipStream_t s, void* dst, const void* src, size_t bytes) {
 int stage_out(int dev, hipStream_t after, void* host, size_t bytes, const StageFill& fill, bool* taken) {
     const OnDevice on(dev);
     HIPCHK(on.error);
+    // few chunks of a small transfer would leave lanes without one, more than
+    // needed cost a launch and an event each
+    const size_t chunk = bytes <= (16u << 20) ? 512u << 10 : bytes <= (64u << 20) ? 1u << 20 : 2u << 20;
     std::unique_lock<std::mutex> lock;
-    Device* const st = lanes_of(dev, bytes, lock);
-    *taken = st != nullptr;
-    if (!st || !bytes) return PF_OK;
-    const size_t chunks = (bytes + STAGE_CHUNK - 1) / STAGE_CHUNK;
-    if (chunks == 1) {  // nothing to overlap: in the stream's own order
-        HIPCHK(fill(after, st->lane[0].chunk[0], 0, bytes));
-        HIPCHK(hipStreamSynchronize(after));
-        memcpy(host, st->lane[0].chunk[0], bytes);
-        return PF_OK;
+    const Ring r = ring_of(dev, bytes, chunk, lock);
+    *taken = r.d != nullptr;
+    if (!r.d || !bytes) return PF_OK;
+    auto issue = [&](size_t c) {
+        const hipError_t e = fill(after, r.at(c), c * chunk, r.len(c));
+        return e != hipSuccess || r.chunks == 1 ? e : hipEventRecord(r.done(c), after);
+    };
+    // a chunk for every lane before the threads start
+    hipError_t e = hipSuccess;
+    for (int w = 0; w < r.lanes && e == hipSuccess; w++) e = issue((size_t)w);
+    if (r.chunks == 1) {
+        if (e == hipSuccess) e = hipStreamSynchronize(after);
+        if (e == hipSuccess) memcpy(host, r.at(0), bytes);
+    } else if (e == hipSuccess) {
+        e = on_lanes(dev, r.lanes, [&](int w) {
+            hipError_t v = hipSuccess;
+            for (size_t c = (size_t)w; c < r.chunks && v == hipSuccess; c += (size_t)r.lanes) {
+                if (c + (size_t)r.lanes < r.chunks) v = issue(c + (size_t)r.lanes);
+                if (v == hipSuccess) v = hipEventSynchronize(r.done(c));
+                if (v == hipSuccess) memcpy((char*)host + c * chunk, r.at(c), r.len(c));
+            }
+            return v;
+        });
     }
-    HIPCHK(hipEventRecord(st->ready, after));
-    const hipError_t e = on_lanes(dev, chunks, [&](int w, int lanes) {
-        Lane& l = st->lane[w];
-        hipError_t r = hipStreamWaitEvent(l.stream, st->ready, 0);
-        auto len = [&](size_t c) { return c + 1 < chunks ? STAGE_CHUNK : bytes - c * STAGE_CHUNK; };
-        auto issue = [&](size_t c, int k) {
-            if (r == hipSuccess) r = fill(l.stream, l.chunk[k], c * STAGE_CHUNK, len(c));
-            if (r == hipSuccess) r = hipEventRecord(l.done[k], l.stream);
-        };
-        int k = 0;
-        issue((size_t)w, 0);
-        for (size_t c = (size_t)w; c < chunks && r == hipSuccess; c += (size_t)lanes, k ^= 1) {
-            if (c + (size_t)lanes < chunks) issue(c + (size_t)lanes, k ^ 1);
-            if (r == hipSuccess) r = hipEventSynchronize(l.done[k]);
-            if (r == hipSuccess) memcpy((char*)host + c * STAGE_CHUNK, l.chunk[k], len(c));
-        }
-        if (r != hipSuccess) (void)hipStreamSynchronize(l.stream);  // nothing writes the chunks any more
-        return r;
-    });
-    if (e != hipSuccess) return fail(PF_ERR_HIP, "transfer to the host: %s", hipGetErrorString(e));
-    return PF_OK;
+    if (e == hipSuccess) return PF_OK;
+    (void)hipStreamSynchronize(after);  // nothing writes the chunks any more
+    return fail(PF_ERR_HIP, "transfer to the host: %s", hipGetErrorString(e));
 }
 
 int stage_in(int dev, hipStream_t after, const void* host, size_t bytes, const StageDrain& drain, bool* taken) {
     const OnDevice on(dev);
     HIPCHK(on.error);
+    const size_t chunk = 2u << 20;  // the host's copy of a smaller one is shorter than its launch
     std::unique_lock<std::mutex> lock;
-    Device* const st = lanes_of(dev, bytes, lock);
-    *taken = st != nullptr;
-    if (!st || !bytes) return PF_OK;
-    const size_t chunks = (bytes + STAGE_CHUNK - 1) / STAGE_CHUNK;
-    if (chunks == 1) {
-        memcpy(st->lane[0].chunk[0], host, bytes);
-        HIPCHK(drain(after, st->lane[0].chunk[0], 0, bytes));
-        HIPCHK(hipStreamSynchronize(after));
-        return PF_OK;
-    }
-    HIPCHK(hipEventRecord(st->ready, after));
-    const hipError_t e = on_lanes(dev, chunks, [&](int w, int lanes) {
-        Lane& l = st->lane[w];
-        hipError_t r = hipStreamWaitEvent(l.stream, st->ready, 0);
-        int k = 0, used = 0;
-        for (size_t c = (size_t)w; c < chunks && r == hipSuccess; c += (size_t)lanes, k ^= 1, used++) {
-            const size_t len = c + 1 < chunks ? STAGE_CHUNK : bytes - c * STAGE_CHUNK;
-            if (used >= 2) r = hipEventSynchronize(l.done[k]);
-            if (r != hipSuccess) break;
-            memcpy(l.chunk[k], (const char*)host + c * STAGE_CHUNK, len);
-            r = drain(l.stream, l.chunk[k], c * STAGE_CHUNK, len);
-            if (r == hipSuccess) r = hipEventRecord(l.done[k], l.stream);
+    const Ring r = ring_of(dev, bytes, chunk, lock);
+    *taken = r.d != nullptr;
+    if (!r.d || !bytes) return PF_OK;
+    const hipError_t e = on_lanes(dev, r.lanes, [&](int w) {
+        hipError_t v = hipSuccess;
+        for (size_t c = (size_t)w; c < r.chunks && v == hipSuccess; c += (size_t)r.lanes) {
+            if (c >= (size_t)(2 * r.lanes)) v = hipEventSynchronize(r.done(c));  // of the slot's last chunk
+            if (v != hipSuccess) break;
+            memcpy(r.at(c), (const char*)host + c * chunk, r.len(c));
+            v = drain(after, r.at(c), c * chunk, r.len(c));
+            if (v == hipSuccess && r.chunks > 1) v = hipEventRecord(r.done(c), after);
         }
-        const hipError_t s = hipStreamSynchronize(l.stream);
-        return r != hipSuccess ? r : s;
+        return v;
     });
-    if (e != hipSuccess) return fail(PF_ERR_HIP, "transfer to the device: %s", hipGetErrorString(e));
-    return PF_OK;
+    const hipError_t s = hipStreamSynchronize(after);  // every chunk is consumed
+    if (e == hipSuccess && s == hipSuccess) return PF_OK;
+    return fail(PF_ERR_HIP, "transfer to the device: %s", hipGetErrorString(e != hipSuccess ? e : s));
 }
 
 int copy_out(int dev, hipStream_t after, void* host, const void* src, size_t bytes) {
@@ -215,7 +204,9 @@ void stage_users(int dev, int change) {
         d.users += change;
         last = change < 0 && d.users == 0;
     }
-    if (last) give_back(d, 1);
+    if (!last) return;
+    std::lock_guard<std::mutex> lock(d.use);
+    if (d.room > STAGE_KEEP) give_back(d);
 }
 
 }  // namespace pf
@@ -223,6 +214,9 @@ void stage_users(int dev, int change) {
 extern "C" int pf_trim(void) {
     int cur = 0;
     if (hipGetDevice(&cur) != hipSuccess) return PF_OK;  // no device, nothing kept
-    for (int i = 0; i < pf::MAX_DEVICES; i++) pf::give_back(pf::g_dev[i], 0);
+    for (pf::Device& d : pf::g_dev) {
+        std::lock_guard<std::mutex> lock(d.use);
+        pf::give_back(d);
+    }
     return PF_OK;
 }

@@ -4,23 +4,33 @@
 // A copy between the device and pageable memory runs at 10 GB/s here: one
 // thread moves every byte through the runtime's own bounce buffer, and a new
 // destination's pages are first touched in that copy.  PCIe moves 57 GB/s.
-// So large transfers go through pinned chunks in a few lanes, each with its
-// own stream, two chunks and a host thread: while one chunk crosses PCIe the
-// thread copies the other.  Fields are packed, and spectra and probe frames
-// copied, by kernels that write the pinned chunks themselves: no device
+// So transfers go through pinned chunks in up to eight lanes, each with two
+// chunks and a host thread: while one chunk crosses PCIe the thread copies the
+// other.  Fields are packed, and spectra and probe frames copied, by kernels
+// that write the pinned chunks themselves, on the caller's stream: no device
 // scratch, no copy command per chunk (2 MiB copy commands from four streams
 // ran at half the kernels' rate).  Three fields of 513 x 513 x 257 nodes (1.6
-// GB) take 32 ms (50 GB/s) against 154; 1.6 MB of a small mesh's fields 0.2
-// against 0.4.  Eight lanes of half a MiB: four of 2 MiB took 40 ms there, and
-// 28 against 18 for the 340 MB of a 16-member batch, whose fields are a few
-// chunks each.
+// GB) take 35 ms (46 GB/s) against 154; 1.6 MB of a small mesh's fields 0.2
+// against 0.27.  Chunks of 512 KiB to 2 MiB by the size: a larger one costs
+// fewer launches (of about 6 us beside a chunk's PCIe time), smaller ones keep
+// the lanes of a short transfer busy.
 //
-// The lanes of a device (2 x STAGE_CHUNK bytes of pinned memory each) are made
-// by the first transfer large enough for them and shared by every context on
-// it.  When the device's last context is destroyed all but the first lane
-// (which a program of many short runs would make again for each) are given
-// back; pf_trim gives back all.  A transfer that finds them taken (another
-// host thread's) copies directly.
+// The lanes have no streams of their own.  With one each the kernels of
+// several chunks overlapped, and 512 KiB chunks were as fast (37 ms there),
+// but a stream takes 0.2 ms to make and one of a process's first four, which
+// bring a hardware queue, 3 ms: the first call then waited longer than it
+// gained.  First calls of a process, ms, pageable copies / lanes with streams
+// / now: a field of 1 MB 6.7 / 6.8 / 0.6, 16 MB 13.9 / 9.3 / 1.8, 64 MB 18 / 11
+// / 5; a transform of 1 MB 2.3 / 8.1 / 1.9, 4 MB 5.9 / 10.6 / 3.2, 16 MB 12 / 11
+// / 4, 64 MB 26 / 15 / 8.
+//
+// The pinned memory of a device is one piece, made by the first transfer and
+// made again when one needs a larger piece (two chunks a lane: 32 MiB at
+// most, 45 us for 8).  It is shared by every context on the device and stays
+// between calls; when the device's last context is destroyed a piece of more
+// than STAGE_KEEP is given back (a program of many short runs would make a
+// smaller one again for each), and pf_trim gives back all.  A transfer that
+// finds it taken (another host thread's) copies directly.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -29,7 +39,7 @@
 namespace pf {
 
 constexpr int STAGE_LANES = 8;
-constexpr size_t STAGE_CHUNK = 512u << 10;
+constexpr size_t STAGE_KEEP = 8u << 20;  // pinned memory that stays when a device has no context left
 
 // Produce bytes [off, off + len) of a transfer at dst (memory the device can
 // write) on stream s, or consume them from src.
@@ -38,7 +48,7 @@ typedef std::function<hipError_t(hipStream_t s, const char* src, size_t off, siz
 
 // Device to host: `fill` produces the bytes, after the work now on stream
 // `after`.  Returns when host[0 .. bytes) is complete.  *taken = false (and
-// nothing done) when the device's chunks are in use.
+// nothing done) when the device's pinned memory is in use.
 int stage_out(int dev, hipStream_t after, void* host, size_t bytes, const StageFill& fill, bool* taken);
 // Host to device: `drain` consumes the bytes, after the work now on stream
 // `after`.  Returns when they are consumed.

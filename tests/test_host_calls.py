@@ -82,3 +82,27 @@ for dev in (0, 1):
         c.close()
     assert count("large_lds@%d" % dev) > 0
 """)
+
+
+def test_transfers_make_no_streams_and_keep_their_pinned_memory(runtime):
+    run(runtime, """
+def plugin_run(cells):
+    c = context(cells)
+    made = count("stream")
+    c.step(2)
+    for f in ("ux", "uy", "uz", "ux_old"):
+        c.get(f)
+    fdtd.dft(np.ones((700, 1000)), nf=500)
+    assert count("stream") == made  # a stream's hardware queue takes milliseconds to make
+    c.close()
+
+plugin_run((90, 60, 40))
+before = count("host_malloc"), count("event")
+assert before[0] <= 2  # one piece, made larger when a transfer first needs it
+for k in range(5):
+    plugin_run((90, 60, 40))
+assert (count("host_malloc"), count("event")) == before
+plugin_run((230, 90, 60))  # 10 MB a field
+fdtd.check(fdtd.load().pf_trim())
+assert count("host_free") == count("host_malloc")
+""")
