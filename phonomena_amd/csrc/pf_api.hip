@@ -501,6 +501,9 @@ int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
     for (int i = 0; i < d->nz - 1; i++) mz += d->fdz[i];
     c->dV = (mx / (d->nx - 1)) * (my / (d->ny - 1)) * (mz / (d->nz - 1));
     for (int e = 0; e < 12; e++) c->mur[e] = d->mur[e];
+    // the audit's partial sums (beside the tables: an audit allocates nothing)
+    c->e_grid = energy_grid(c->nx, c->plane);
+    HIPCHK(hipMalloc((void**)&c->e_partials, 2 * sizeof(double) * (size_t)(c->e_grid.blocks + 1)));
 
     // source table (FP64 on the device) and step counter
     c->wave_len = d->wave_len;
@@ -540,7 +543,6 @@ void pf::ctx_free(pf_ctx* c) {
     F(c->dpx); F(c->dpy); F(c->dpz);
     F(c->mat64); F(c->rho64); F(c->fx64); F(c->fy64); F(c->fz64); F(c->sx64); F(c->sy64); F(c->sz64);
     F(c->wave); F(c->d_step); F(c->ring); F(c->d_frame); F(c->e_partials);
-    if (c->e_out) (void)hipHostFree(c->e_out);
     F(c->scratch);
     if (c->snap_stream) (void)hipStreamSynchronize(c->snap_stream);  // no copy in flight
     F(c->snap_dev);
@@ -1219,17 +1221,9 @@ static int launch_energy(pf_ctx* c, const EnergyArgs& ea, dim3 grid, hipStream_t
 extern "C" int pf_energy(pf_ctx* c, double* out) {
     if (!c || !out) return fail(PF_ERR_ARG, "NULL argument");
     hipStream_t s = c->batch ? c->batch_stream : c->stream;
-    // about 8 blocks per CU, 4 to ENERGY_XCHUNK planes each
-    const long long per = (c->plane + ENERGY_CELLS - 1) / ENERGY_CELLS;
-    long long want = (2048 + per - 1) / per;
-    if (want > (c->nx + 3) / 4) want = (c->nx + 3) / 4;
-    int xc = (int)((c->nx + want - 1) / want);
-    if (xc > ENERGY_XCHUNK) xc = ENERGY_XCHUNK;
-    const long long blocks = per * ((c->nx + xc - 1) / xc);
+    const long long blocks = c->e_grid.blocks;
     if (blocks > 0x7fffffffLL) return fail(PF_ERR_ARG, "mesh too large for the energy audit");
     const dim3 grid((unsigned)blocks);
-    if (!c->e_partials) HIPCHK(hipMalloc((void**)&c->e_partials, 2 * sizeof(double) * (size_t)blocks));
-    if (!c->e_out) HIPCHK(hipHostMalloc((void**)&c->e_out, 2 * sizeof(double), hipHostMallocDefault));
     EnergyArgs ea;
     ea.mat = (const double*)c->mat64;
     ea.rho = (const double*)c->rho64;
@@ -1241,17 +1235,31 @@ extern "C" int pf_energy(pf_ctx* c, double* out) {
     }
     ea.dt = c->dt;
     ea.w_prev = c->step > 0 ? c->wave + (c->step - 1) : nullptr;
-    ea.xchunk = xc;
-    ea.per = (unsigned)per;
+    ea.xchunk = c->e_grid.xchunk;
+    ea.per = (unsigned)c->e_grid.per;
     int rc;
     if (c->precision == PF_FP64) rc = launch_energy<double, false>(c, ea, grid, s);
     else if (c->precision == PF_FP32) rc = launch_energy<float, false>(c, ea, grid, s);
     else rc = launch_energy<float, true>(c, ea, grid, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(1024), 0, s, (const double*)c->e_partials, blocks, c->e_out);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(s));  // the sums land in pinned host memory
-    *out = 0.5 * c->dV * (c->e_out[0] + c->e_out[1]);
+    // the two sums, into pinned memory where there is some to be had
+    const double* const parts = c->e_partials;
+    double h[2];
+    bool taken = false;
+    rc = stage_out(c->dev, s, h, sizeof h, [=](hipStream_t q, char* dst, size_t, size_t) {
+        hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(1024), 0, q, parts, blocks, (double*)dst);
+        return hipGetLastError();
+    }, &taken);
+    if (!taken) {
+        double* const sums = c->e_partials + 2 * blocks;
+        hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(1024), 0, s, parts, blocks, sums);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(h, sums, sizeof h, hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+    } else if (rc) {
+        return rc;
+    }
+    *out = 0.5 * c->dV * (h[0] + h[1]);
     return PF_OK;
 }
 

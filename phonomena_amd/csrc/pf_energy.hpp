@@ -15,8 +15,10 @@
 // FP32, 130 in FP64 (166, 95 and 150 with the z neighbours loaded and decoded
 // again), against 680, 621 and 453 with levels widened to FP64 arrays by
 // six launches first and a grid-stride kernel with 64-bit index divisions and
-// quotients per node; 20 us on small meshes (81 and 40).  The relative error
-// against a 64-bit restatement is the same (2e-16 to 8e-16 in FP64).
+// quotients per node; 21 us on small meshes (81 in FP32C, 42 in FP64).  A
+// context's first call costs 3 us more: the partial sums are allocated with it
+// and the two sums pass through the transfers' pinned memory (allocated by the
+// first call they cost 26 to 40 us there).  The relative error against a 64-bit restatement is the same (2e-16 to 8e-16 in FP64).
 //
 // Per-thread sums, a wavefront/LDS tree per block, then one block adds the
 // block partials in a fixed order, so the result is deterministic.
@@ -43,6 +45,18 @@ PF_DEV double warp_sum(double v) {
 
 constexpr int ENERGY_XCHUNK = 32;  // most planes per block
 constexpr int ENERGY_CELLS = 4 * 62;  // cells per block: a wave's outer lanes are its neighbours' cells
+
+// About 8 blocks per CU, 4 to ENERGY_XCHUNK planes each.
+inline EnergyGrid energy_grid(int nx, long long plane) {
+    EnergyGrid g;
+    g.per = (plane + ENERGY_CELLS - 1) / ENERGY_CELLS;
+    long long want = (2048 + g.per - 1) / g.per;
+    if (want > (nx + 3) / 4) want = (nx + 3) / 4;
+    g.xchunk = (int)((nx + want - 1) / want);
+    if (g.xchunk > ENERGY_XCHUNK) g.xchunk = ENERGY_XCHUNK;
+    g.blocks = g.per * ((nx + g.xchunk - 1) / g.xchunk);
+    return g;
+}
 
 // One level's value of a component at cell a of its array.
 template <bool COMP, class R>

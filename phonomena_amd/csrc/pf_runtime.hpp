@@ -33,6 +33,11 @@ struct BlockMap {
     int ntx, nty, ntz, steps, threads;
 };
 constexpr int BLOCK_MAX_STEPS = 4;
+// Blocks of an energy audit: `per` a chunk of xchunk planes (pf_energy.hpp).
+struct EnergyGrid {
+    long long per, blocks;
+    int xchunk;
+};
 }  // namespace pf
 
 // One mesh on one device.  Time levels of the displacement components are
@@ -96,9 +101,8 @@ struct pf_ctx {
     int every = 0, cap = 0;
     double* ring = nullptr;
     long long* d_frame = nullptr;  // [0] frames recorded; [1], as an int: blocks done in the probe launch
-    // energy audit, allocated by its first call: the two sums (pinned host
-    // memory) and the blocks' partial sums
-    double* e_out = nullptr;
+    // energy audit: the blocks' partial sums, then room for the two sums
+    pf::EnergyGrid e_grid = {};
     double* e_partials = nullptr;
     void* scratch = nullptr;
     size_t scratch_bytes = 0;

@@ -198,15 +198,20 @@ int copy_in(int dev, hipStream_t after, void* dst, const void* host, size_t byte
 void stage_users(int dev, int change) {
     if (dev < 0 || dev >= MAX_DEVICES) return;
     Device& d = g_dev[dev];
-    bool last;
+    bool first, last;
     {
         std::lock_guard<std::mutex> lock(d.count);
+        first = change > 0 && d.users == 0;
         d.users += change;
         last = change < 0 && d.users == 0;
     }
-    if (!last) return;
-    std::lock_guard<std::mutex> lock(d.use);
-    if (d.room > STAGE_KEEP) give_back(d);
+    if (!first && !last) return;
+    std::unique_lock<std::mutex> lock(d.use, std::try_to_lock);
+    if (!lock.owns_lock()) return;  // a transfer without a context runs
+    if (last && d.room > STAGE_KEEP) give_back(d);
+    // the first fetch or audit of the device's first context finds it made
+    const OnDevice on(dev);
+    if (first && on.error == hipSuccess && reserve(d, 512u << 10) != hipSuccess) (void)hipGetLastError();
 }
 
 }  // namespace pf

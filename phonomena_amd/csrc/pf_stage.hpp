@@ -24,9 +24,9 @@
 // / 5; a transform of 1 MB 2.3 / 8.1 / 1.9, 4 MB 5.9 / 10.6 / 3.2, 16 MB 12 / 11
 // / 4, 64 MB 26 / 15 / 8.
 //
-// The pinned memory of a device is one piece, made by the first transfer and
-// made again when one needs a larger piece (two chunks a lane: 32 MiB at
-// most, 45 us for 8).  It is shared by every context on the device and stays
+// The pinned memory of a device is one piece, of 512 KiB with its first
+// context and made again when a transfer needs a larger one (two chunks a
+// lane: 32 MiB at most; 8 MiB take 45 us).  It is shared by every context on the device and stays
 // between calls; when the device's last context is destroyed a piece of more
 // than STAGE_KEEP is given back (a program of many short runs would make a
 // smaller one again for each), and pf_trim gives back all.  A transfer that
