@@ -18,7 +18,8 @@
 // quotients per node; 21 us on small meshes (81 in FP32C, 42 in FP64).  A
 // context's first call costs 3 us more: the partial sums are allocated with it
 // and the two sums pass through the transfers' pinned memory (allocated by the
-// first call they cost 26 to 40 us there).  The relative error against a 64-bit restatement is the same (2e-16 to 8e-16 in FP64).
+// first call they cost 26 to 40 us there).  The relative error against a
+// 64-bit restatement is the same (2e-16 to 8e-16 in FP64).
 //
 // Per-thread sums, a wavefront/LDS tree per block, then one block adds the
 // block partials in a fixed order, so the result is deterministic.

@@ -34,17 +34,30 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <functional>
-
 namespace pf {
 
 constexpr int STAGE_LANES = 8;
 constexpr size_t STAGE_KEEP = 8u << 20;  // pinned memory that stays when a device has no context left
 
 // Produce bytes [off, off + len) of a transfer at dst (memory the device can
-// write) on stream s, or consume them from src.
-typedef std::function<hipError_t(hipStream_t s, char* dst, size_t off, size_t len)> StageFill;
-typedef std::function<hipError_t(hipStream_t s, const char* src, size_t off, size_t len)> StageDrain;
+// write) on stream s, or consume them from src: a reference to the caller's
+// function object, for the length of the call (std::function would allocate,
+// and throw through a C entry).
+template <class P>
+class StageFn {
+    const void* obj;
+    hipError_t (*call)(const void* obj, hipStream_t s, P at, size_t off, size_t len);
+
+public:
+    template <class F>
+    StageFn(const F& f)
+        : obj(&f), call([](const void* o, hipStream_t s, P at, size_t off, size_t len) -> hipError_t {
+              return (*(const F*)o)(s, at, off, len);
+          }) {}
+    hipError_t operator()(hipStream_t s, P at, size_t off, size_t len) const { return call(obj, s, at, off, len); }
+};
+typedef StageFn<char*> StageFill;
+typedef StageFn<const char*> StageDrain;
 
 // Device to host: `fill` produces the bytes, after the work now on stream
 // `after`.  Returns when host[0 .. bytes) is complete.  *taken = false (and

@@ -33,7 +33,15 @@ static float (*g_elapsed)(int, int) = nullptr;
 struct Call { Dim3 grid, block; size_t lds; Stream* stream; };
 static thread_local Call t_call;
 
+// The stand-in's own allocations never fail.
+static thread_local int t_inside = 0;
+struct Inside {
+    Inside() { t_inside++; }
+    ~Inside() { t_inside--; }
+};
+
 static void count(const char* what, int dev) {
+    Inside in;
     std::lock_guard<std::mutex> l(g_lock);
     g_count[what]++;
     g_count[std::string(what) + "@" + std::to_string(dev)]++;
@@ -49,7 +57,7 @@ long long host_count(const char* what) {
 int host_launches() { return (int)g_launches.size(); }
 const char* host_launch(int i) { return g_launches[(size_t)i].c_str(); }
 void host_fail_host_malloc(int on) { g_fail_host_malloc = on; }
-void host_fail_new(int after) { g_fail_new = after; }
+void host_fail_new(int on) { g_fail_new = on; }
 void host_elapsed(float (*f)(int, int)) { g_elapsed = f; }
 
 // ---- devices ----
@@ -72,6 +80,7 @@ hipError_t hipGetLastError() {
 static hipError_t take(void** p, size_t n, const char* what) {
     *p = calloc(1, n ? n : 1);
     count(what, t_dev);
+    Inside in;
     std::lock_guard<std::mutex> l(g_lock);
     g_owner[*p] = t_dev;
     return 0;
@@ -98,6 +107,7 @@ hipError_t hipMemcpy2DAsync(void*, size_t, const void*, size_t, size_t, size_t, 
 
 // ---- streams and events ----
 hipError_t hipStreamCreateWithFlags(Stream** s, unsigned) {
+    Inside in;
     count("stream", t_dev);
     *s = new Stream{t_dev};
     return 0;
@@ -106,6 +116,7 @@ hipError_t hipStreamDestroy(Stream* s) { count("stream_destroy", s->dev); delete
 hipError_t hipStreamSynchronize(Stream*) { return 0; }
 hipError_t hipStreamWaitEvent(Stream*, Event*, unsigned) { return 0; }
 hipError_t hipEventCreateWithFlags(Event** e, unsigned) {
+    Inside in;
     count("event", t_dev);
     *e = new Event{t_dev, 0};
     return 0;
@@ -136,12 +147,14 @@ hipError_t __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* lds, Stream** s) 
     return 0;
 }
 hipError_t hipFuncSetAttribute(const void* f, int, int v) {
+    Inside in;
     std::lock_guard<std::mutex> l(g_lock);
     g_lds[{f, t_dev}] = v;
     return 0;
 }
 hipError_t hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t lds, Stream* s) {
     const int dev = dev_of(s);
+    Inside in;
     count("launch", dev);
     if (lds > 65536) count("large_lds", dev);
     std::lock_guard<std::mutex> l(g_lock);
@@ -161,13 +174,9 @@ hipError_t hipGraphExecDestroy(void*) { return 0; }
 hipError_t hipGraphDestroy(void*) { return 0; }
 }
 
-// Allocations of the library's C++ code fail from the n-th on after
-// host_fail_new(n).
+// Allocations of the library's C++ code fail after host_fail_new(1).
 void* operator new(size_t n) {
-    if (g_fail_new > 0 && --g_fail_new == 0) {
-        g_fail_new = 1;  // and every later one
-        throw std::bad_alloc();
-    }
+    if (g_fail_new && !t_inside) throw std::bad_alloc();
     if (void* p = malloc(n ? n : 1)) return p;
     throw std::bad_alloc();
 }

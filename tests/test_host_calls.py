@@ -126,3 +126,26 @@ for cells in ((40, 30, 20), (70, 80, 30)):
     assert allocations() == made
     c.close()
 """ % (not pinned, precision))
+
+
+@pytest.mark.parametrize("pinned", [True, False])
+def test_transfers_and_audits_without_host_memory_do_not_throw(runtime, pinned):
+    """No C++ exception may leave a C entry: without memory for a thread or a
+    function object a transfer runs on the caller's thread."""
+    run(runtime, """
+hip.host_fail_host_malloc(%d)
+c = context((120, 40, 40), probe=(0, 1, 120, 0, 1, 40), every=1)
+a = np.zeros(c._shapes["ux"])
+x = np.ones((900, 1000))
+c.get("ux")
+hip.host_fail_new(1)
+for f in ("ux", "uz_old"):
+    c.get(f)
+c.set("ux", a)
+c.step(20)
+c.probes()
+c.energy()
+fdtd.dft(x, nf=500)
+hip.host_fail_new(0)
+c.close()
+""" % (not pinned))
