@@ -314,10 +314,15 @@ int sweep_grid_s(pf_batch* b, int tj, int tz) {
 }
 
 template <class R, int MODE>
+int sweep_grid_t(pf_batch* b, int tj, int tz) {
+    return b->sponge == 1 ? sweep_grid_s<R, MODE, true>(b, tj, tz) : sweep_grid_s<R, MODE, false>(b, tj, tz);
+}
+
+template <class R, int MODE>
 int build_t(pf_batch* b) {
     int tj, tz;
     batch_shape(b, tj, tz);
-    int rc = b->sponge == 1 ? sweep_grid_s<R, MODE, true>(b, tj, tz) : sweep_grid_s<R, MODE, false>(b, tj, tz);
+    int rc = sweep_grid_t<R, MODE>(b, tj, tz);
     if (rc) return rc;
     const int tx = b->tile_x ? b->tile_x : default_xchunk(b, tj, tz);
     const int nmem = (int)b->members.size();
@@ -408,7 +413,7 @@ int build_t(pf_batch* b) {
 // The FP64 flavour is the one all members allow: reciprocal products, exact
 // quotients, else divisions (all the same bits).  16 members of 14.2 M nodes,
 // us a step: 286, 355 (at a spacing of 0.3), 399; 5 of 1.4 M: 49, 65, 71.
-int build(pf_batch* b) {
+void choose_mode(pf_batch* b) {
     bool recip = true, quot = true;
     for (const pf_ctx* c : b->members) {
         recip = recip && c->recip;
@@ -419,12 +424,28 @@ int build(pf_batch* b) {
               : recip                   ? MODE_FP64P
               : quot                    ? MODE_FP64Q
                                         : MODE_FP64;
+}
+
+int build(pf_batch* b) {
+    choose_mode(b);
     switch (b->mode) {
         case MODE_FP64: return build_t<double, MODE_FP64>(b);
         case MODE_FP64P: return build_t<double, MODE_FP64P>(b);
         case MODE_FP64Q: return build_t<double, MODE_FP64Q>(b);
         case MODE_FP32: return build_t<float, MODE_FP32>(b);
         default: return build_t<float, MODE_FP32C>(b);
+    }
+}
+
+// Blocks of the sweep with this shape (b->grid).
+int shape_grid(pf_batch* b, int tj, int tz) {
+    choose_mode(b);
+    switch (b->mode) {
+        case MODE_FP64: return sweep_grid_t<double, MODE_FP64>(b, tj, tz);
+        case MODE_FP64P: return sweep_grid_t<double, MODE_FP64P>(b, tj, tz);
+        case MODE_FP64Q: return sweep_grid_t<double, MODE_FP64Q>(b, tj, tz);
+        case MODE_FP32: return sweep_grid_t<float, MODE_FP32>(b, tj, tz);
+        default: return sweep_grid_t<float, MODE_FP32C>(b, tj, tz);
     }
 }
 
@@ -613,14 +634,18 @@ extern "C" int pf_batch_autotune(pf_batch* b, int32_t trial_steps, int32_t* tile
     if (b->members.empty()) return fail(PF_ERR_STATE, "batch has no members");
     struct Cand { int tj, tz, tx; };
     std::vector<Cand> cands;
-    const int xs[] = {16, 32, 64, 128};
-    if (b->precision == PF_FP64) {
-        for (int tx : xs) { cands.push_back({8, 32, tx}); cands.push_back({16, 32, tx}); cands.push_back({8, 64, tx}); }
-    } else {
-        for (int tx : xs) {
-            cands.push_back({16, 64, tx}); cands.push_back({8, 64, tx});
-            cands.push_back({32, 32, tx}); cands.push_back({16, 32, tx}); cands.push_back({8, 32, tx});
-        }
+    const int shapes[][2] = {{16, 64}, {8, 64}, {32, 32}, {16, 32}, {8, 32}};
+    const int shapes64[][2] = {{8, 32}, {16, 32}, {8, 64}};
+    const bool f64 = b->precision == PF_FP64;
+    for (int q = 0; q < (f64 ? 3 : 5); q++) {
+        const int* const sh = f64 ? shapes64[q] : shapes[q];
+        // the shape's default chunk among them: below 32 planes, where it is
+        // none of the others, it takes the place of 128, whose items would
+        // leave most blocks without one
+        int rc = shape_grid(b, sh[0], sh[1]);
+        if (rc) return rc;
+        const int own = default_xchunk(b, sh[0], sh[1]);
+        for (int tx : {16, 32, 64, own == 16 || own == 32 ? 128 : own}) cands.push_back({sh[0], sh[1], tx});
     }
     // every candidate runs 1 untimed + trial_steps timed steps of real work
     long long room = 0;

@@ -149,3 +149,33 @@ fdtd.dft(x, nf=500)
 hip.host_fail_new(0)
 c.close()
 """ % (not pinned))
+
+
+@pytest.mark.parametrize("precision,shapes,default", [("fp32c", 5, (16, 32)), ("fp32", 5, (16, 32)),
+                                                      ("fp64", 3, (8, 32))])
+@pytest.mark.parametrize("cells,chunk", [((60, 50, 24), 8), ((170, 170, 80), 32)])
+def test_the_autotuner_tries_the_default(runtime, precision, shapes, default, cells, chunk):
+    """The candidates, one by one: the stand-in's clock makes each the
+    fastest in turn.  Their number is the steps a caller has to leave for them."""
+    run(runtime, """
+FASTEST = ctypes.CFUNCTYPE(ctypes.c_float, ctypes.c_int, ctypes.c_int)
+found = set()
+ctxs = [context(%r, precision=%r, steps=2000) for _ in range(3)]
+b = fdtd.Batch(%r)
+for c in ctxs:
+    b.add(c)
+n = 4 * %d
+for k in range(n):
+    calls = [0]
+    def clock(_a, _b):
+        calls[0] += 1
+        return 1.0 if calls[0] == k + 1 else 2.0
+    f = FASTEST(clock)
+    hip.host_elapsed(f)
+    before = ctxs[0].steps_done
+    best = b.autotune(trial_steps=1)
+    assert calls[0] == n and ctxs[0].steps_done - before == 2 * n
+    found.add((best["tile_j"], best["tile_z"], best["tile_x"]))
+assert len(found) == n
+assert %r in found, sorted(found)
+""" % (cells, precision, precision, shapes, default + (chunk,)))
