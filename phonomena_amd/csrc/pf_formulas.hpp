@@ -181,8 +181,10 @@ PF_DEV R div3_uz_surface(R d1, R g1, R d2, R g2, R t3k1, R t3k0, R fz0) {
 }
 
 // ---- leapfrog ---------------------------------------------------------------
-// u_new = 2 u - u_old + coef * div (base_solver.py:441-443); 2 u is exact, so
-// the difference takes one fused operation.  With a damping
+// u_new = 2 u - u_old + coef * div (base_solver.py:441-443).  In FP32 the
+// difference takes one fused operation (2 u is exact, and where it would
+// overflow a difference that does not is kept); in FP64 two, since 2 u
+// overflows there in the reference (fused it measured no faster).  With a damping
 // term s > 0 (sponge extension): ((2u - (1-s) u_old) + coef*div) / (1+s);
 // in FP32 the division is a product with the hardware reciprocal of 1+s
 // (v_rcp_f32, within 1 ulp; one per node, shared by its three components:
@@ -196,11 +198,11 @@ PF_DEV R leap(R u, R uo, R coef, R dv, R s) {
         if constexpr (SPONGE) {
             // off the absorbing layer s = 0: (1 - 0) u_old = u_old and
             // x / (1 + 0) = x exactly, so the division is skipped there
-            R r = mad(R(2), u, -((1 - s) * uo)) + coef * dv;
+            R r = 2 * u - (1 - s) * uo + coef * dv;
             if (s != R(0)) r = r / (1 + s);
             return r;
         }
-        else return mad(R(2), u, -uo) + coef * dv;
+        else return 2 * u - uo + coef * dv;
     } else {
         if constexpr (SPONGE) return mad(coef, dv, mad(R(2), u, -((1 - s) * uo))) * __builtin_amdgcn_rcpf(1 + s);
         else return mad(coef, dv, mad(R(2), u, -uo));
