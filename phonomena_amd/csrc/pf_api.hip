@@ -13,6 +13,7 @@
 #include "../../include/phonofdtd.h"
 #include "pf_energy.hpp"
 #include "pf_kernels.hpp"
+#include "pf_quotient.hpp"
 #include "pf_runtime.hpp"
 #include "pf_strip.hpp"
 #include "pf_fused.hpp"
@@ -143,38 +144,6 @@ static bool pow2_spacings(const pf_desc* d) {
             int e = 0;
             const double f = std::frexp(t[a][i], &e);
             if (!std::isfinite(t[a][i]) || f != 0.5 || e < -1000 || e > 1000) return false;
-        }
-    return true;
-}
-
-// Whether quotient()'s three operations (pf_formulas.hpp) give RN(a / h) for
-// every dividend a.  With h = B 2^e and a = A 2^f, B and A integers of 53 bits,
-// a quotient near a rounding boundary M (an odd integer of 54 bits, half an
-// ulp its unit) has A 2^w = B M + t, w = 53 or 54, with |t| / 2B its distance
-// in ulp.  The operations' error before the last rounding is below 2^-51 ulp
-// (1.5 ulp of the first quotient times the relative errors of 1 / h and of the
-// remainder), so only |t| <= 8 matters; the dividends of |t| <= 16 are found
-// from M = -t / B mod 2^w and tried.
-static bool quotient_exact(double h) {
-    int e = 0;
-    const uint64_t B = (uint64_t)std::ldexp(std::frexp(h, &e), 53);
-    const double b = (double)B, y = 1.0 / b;
-    const int z = __builtin_ctzll(B);
-    if (z > 4) return true;  // then |t| is 0 or above 16
-    uint64_t inv = B >> z;   // (B / 2^z)^-1 mod 2^64, by Newton's steps
-    for (int k = 0; k < 6; k++) inv *= 2 - (B >> z) * inv;
-    for (int w = 53; w <= 54; w++)
-        for (int t = -16; t <= 16; t++) {
-            if (t == 0 || t % (1 << z)) continue;
-            const uint64_t mod = 1ull << (w - z), lo = 1ull << 53;
-            uint64_t M = ((uint64_t)(int64_t)(-t / (1 << z)) * inv) & (mod - 1);
-            if (M < lo) M += (lo - M + mod - 1) / mod * mod;
-            for (; M < 2 * lo; M += mod) {
-                const uint64_t A = (uint64_t)(((unsigned __int128)B * M + (__int128)t) >> w);
-                if (A < lo / 2 || A >= lo) continue;
-                const double a = (double)A, q = a * y;
-                if (std::fma(std::fma(-b, q, a), y, q) != a / b) return false;
-            }
         }
     return true;
 }

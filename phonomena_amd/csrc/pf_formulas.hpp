@@ -65,7 +65,7 @@ template <class H, class R> PF_DEV H spacing(R h, R y) {
 // corrected sum differs from a / h by less than 2^-51 ulp before it is
 // rounded, and RN of it is RN(a / h) unless a / h is that near a rounding
 // boundary.  For a given h only a few dividends come so near; the host tries
-// the three operations on all of them (quotient_exact, pf_api.hip) and leaves
+// the three operations on all of them (pf_quotient.hpp) and leaves
 // a mesh with a spacing that fails to the divisions (none was found among
 // 2 x 10^6 random spacings).  This holds while nothing on the way underflows
 // or overflows, which follows from the displacements alone (in_range): with
