@@ -2,10 +2,12 @@
 // cycle, stepping, field transfer, probes, energy audit, profiling.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -148,18 +150,17 @@ static bool pow2_spacings(const pf_desc* d) {
     return true;
 }
 
-// Whether quotient() (pf_formulas.hpp) is exact on this mesh for every
-// displacement in its range: spacings within 2^-60 .. 2^20 that quotient_exact
-// holds for, stiffness entries 0 or within 2^-20 .. 2^100.
-static bool quotients_allowed(const pf_desc* d) {
-    const double* t[6] = {d->fdx, d->fdy, d->fdz, d->sdx, d->sdy, d->sdz};
-    const int n[6] = {d->nx - 1, d->ny - 1, d->nz - 1, d->nx - 2, d->ny - 2, d->nz - 2};
-    for (int a = 0; a < 6; a++)
-        for (int i = 0; i < n[a]; i++) {
-            const double h = t[a][i];
-            if (i > 0 && h == t[a][i - 1]) continue;
-            if (!(h >= 0x1p-60 && h <= 0x1p20) || !quotient_exact(h)) return false;
-        }
+// quotient() (pf_formulas.hpp) is exact on a mesh for every displacement in its
+// range if its spacings are within 2^-60 .. 2^20 and hold quotient_exact, and
+// its stiffness entries are 0 or within 2^-20 .. 2^100.
+static bool spacings_allow_quotients(const double* t, int n) {
+    for (int i = 0; i < n; i++) {
+        if (i > 0 && t[i] == t[i - 1]) continue;
+        if (!(t[i] >= 0x1p-60 && t[i] <= 0x1p20) || !quotient_exact(t[i])) return false;
+    }
+    return true;
+}
+static bool stiffnesses_allow_quotients(const pf_desc* d) {
     for (int r = 0; r < d->n_materials; r++)
         for (int q = 0; q < 12; q++) {
             const double v = std::fabs(d->materials[r * 13 + q]);
@@ -168,11 +169,48 @@ static bool quotients_allowed(const pf_desc* d) {
     return true;
 }
 
+// The six spacing tables of an FP64 context on the device, their lengths and
+// where their reciprocals go.
+struct SpacingTables {
+    const void* h[6];
+    int n[6];
+    void** y[6];
+    explicit SpacingTables(pf_ctx* c)
+        : h{c->fx, c->fy, c->fz, c->sx, c->sy, c->sz},
+          n{c->nx - 1, c->ny - 1, c->nz - 1, c->nx - 2, c->ny - 2, c->nz - 2},
+          y{&c->rfx, &c->rfy, &c->rfz, &c->rsx, &c->rsy, &c->rsz} {}
+};
+
+// For a batch, which marches its members: whether this one, which steps in
+// blocks by itself (with divisions), may take quotients, and the tables for
+// them.  Where they cannot be had it divides.
+void pf::take_quotients(pf_ctx* c) {
+    if (!c->quot_open) return;
+    c->quot_open = false;
+    const OnDevice on(c->dev);
+    if (on.error != hipSuccess) return;
+    const SpacingTables t(c);
+    const int most = std::max(c->nx, std::max(c->ny, c->nz));
+    const std::unique_ptr<double[]> v(new (std::nothrow) double[(size_t)most]);
+    if (!v) return;
+    hipError_t e = hipSuccess;
+    for (int a = 0; a < 6 && e == hipSuccess; a++) {
+        const size_t bytes = (size_t)t.n[a] * sizeof(double);
+        e = hipMemcpy(v.get(), t.h[a], bytes, hipMemcpyDeviceToHost);
+        if (e == hipSuccess && !spacings_allow_quotients(v.get(), t.n[a])) return;
+        for (int i = 0; i < t.n[a]; i++) v[(size_t)i] = 1.0 / v[(size_t)i];
+        if (e == hipSuccess && !*t.y[a]) e = hipMalloc(t.y[a], bytes);
+        if (e == hipSuccess) e = hipMemcpy(*t.y[a], v.get(), bytes, hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess) c->quot = true;
+    else (void)hipGetLastError();
+}
+
 template <class R>
 static int create_tables(pf_ctx* c, const pf_desc* d) {
     const bool exact = d->precision == PF_FP64;
     int rc;
-    if (exact) {
+    if (c->recip || c->quot) {
         if ((rc = upload_table(&c->rfx, spacing_table<double>(d->fdx, d->nx - 1, true)))) return rc;
         if ((rc = upload_table(&c->rfy, spacing_table<double>(d->fdy, d->ny - 1, true)))) return rc;
         if ((rc = upload_table(&c->rfz, spacing_table<double>(d->fdz, d->nz - 1, true)))) return rc;
@@ -397,8 +435,17 @@ int pf::ctx_init(pf_ctx* c, const pf_desc* d) {
     // the FP64 one-step tiled sweep and block steps on power-of-two spacings
     // multiply by exact reciprocals (MODE_FP64P)
     c->recip = d->precision == PF_FP64 && c->kernel == PF_KERNEL_TILED && pow2_spacings(d);
-    c->quot = d->precision == PF_FP64 && c->kernel == PF_KERNEL_TILED && !c->recip && quotients_allowed(d);
     if (d->kernel == PF_KERNEL_AUTO && c->kernel == PF_KERNEL_TILED && c->shape_open && c->tile_x == 0) block_plan(c);
+    // else they take quotients where they are exact; trying the spacings costs
+    // 0.8 us for each, so a mesh that steps in blocks, with divisions, leaves it
+    // to the batch that it may join
+    c->quot_open = d->precision == PF_FP64 && c->kernel == PF_KERNEL_TILED && !c->recip && stiffnesses_allow_quotients(d);
+    if (c->quot_open && !c->block_steps) {
+        c->quot_open = false;
+        c->quot = spacings_allow_quotients(d->fdx, d->nx - 1) && spacings_allow_quotients(d->fdy, d->ny - 1) &&
+                  spacings_allow_quotients(d->fdz, d->nz - 1) && spacings_allow_quotients(d->sdx, d->nx - 2) &&
+                  spacings_allow_quotients(d->sdy, d->ny - 2) && spacings_allow_quotients(d->sdz, d->nz - 2);
+    }
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
 
     // fields: two levels (four for the two-step sweep) x three components
@@ -560,7 +607,7 @@ Mesh<R> pf::make_view(const pf_ctx* c, int cur, int old, int nxt) {
     m.sx0 = (R)(exact ? c->s0[0] : 1.0 / c->s0[0]);
     m.sy0 = (R)(exact ? c->s0[1] : 1.0 / c->s0[1]);
     m.sz0 = (R)(exact ? c->s0[2] : 1.0 / c->s0[2]);
-    if (exact) {
+    if (c->recip || c->quot) {
         m.rfx = (const R*)c->rfx; m.rfy = (const R*)c->rfy; m.rfz = (const R*)c->rfz;
         m.rsx = (const R*)c->rsx; m.rsy = (const R*)c->rsy; m.rsz = (const R*)c->rsz;
         m.rfx0 = (R)(1.0 / c->f0[0]); m.rfy0 = (R)(1.0 / c->f0[1]); m.rfz0 = (R)(1.0 / c->f0[2]);

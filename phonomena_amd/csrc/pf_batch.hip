@@ -579,6 +579,7 @@ extern "C" int pf_batch_add(pf_batch* b, pf_ctx* c) {
         return fail(PF_ERR_ARG, "all members of a batch either have an absorbing layer or none");
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
+    take_quotients(c);
     b->sponge = sp;
     b->members.push_back(c);
     c->batch = b;

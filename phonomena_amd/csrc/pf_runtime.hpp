@@ -84,9 +84,10 @@ struct pf_ctx {
     void *dpx = nullptr, *dpy = nullptr, *dpz = nullptr;
     // FP64: the reciprocals of the spacing tables, which fx.. keep.  recip:
     // every spacing is a power of two, so the tiled sweep and block steps
-    // multiply by them (MODE_FP64P); quot: otherwise they take exact quotients
-    // from them (MODE_FP64Q).
-    bool recip = false, quot = false;
+    // multiply by them (MODE_FP64P); quot: otherwise the tiled sweep takes exact
+    // quotients from them (MODE_FP64Q); quot_open: it might, the spacings are
+    // not tried (take_quotients).
+    bool recip = false, quot = false, quot_open = false;
     void *rfx = nullptr, *rfy = nullptr, *rfz = nullptr, *rsx = nullptr, *rsy = nullptr, *rsz = nullptr;
     void *mat64 = nullptr, *rho64 = nullptr, *fx64 = nullptr, *fy64 = nullptr, *fz64 = nullptr,
          *sx64 = nullptr, *sy64 = nullptr, *sz64 = nullptr;
@@ -159,6 +160,7 @@ struct OnDevice {
 
 int ctx_init(pf_ctx* c, const pf_desc* d);
 void ctx_free(pf_ctx* c);
+void take_quotients(pf_ctx* c);
 // View of a step from level `cur` (n) and `old` (n-1) into level `out`.
 template <class R>
 Mesh<R> make_view(const pf_ctx* c, int cur, int old, int out);

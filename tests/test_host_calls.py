@@ -179,3 +179,32 @@ for k in range(n):
 assert len(found) == n
 assert %r in found, sorted(found)
 """ % (cells, precision, precision, shapes, default + (chunk,)))
+
+
+def test_reciprocals_are_made_for_the_kernels_that_read_them(runtime):
+    run(runtime, """
+def made(cells, kernel, spacing, tune=True):
+    before = count("malloc")
+    c = context(cells, kernel=kernel, spacing=spacing, tune=tune)
+    return c, count("malloc") - before
+
+small, large = (30, 24, 12), (90, 70, 60)
+plain = made(large, "naive", 0.3)[1]
+assert made(large, "strip", 0.3)[1] == plain
+assert made(large, "tiled", 0.3)[1] == plain + 6     # exact quotients
+assert made(large, "tiled", 0.5)[1] == plain + 6     # reciprocal products
+c, n = made(small, "auto", 0.3)                      # block steps with divisions: two more levels
+assert n == plain + 2
+c.step(4)
+assert "k_block_stepsIdLi0E" in launches()[-1]
+# a batch marches its members, with quotients
+d, _ = made(large, "auto", 0.7, tune=False)
+b = fdtd.Batch("fp64")
+for m in (c, d):
+    b.add(m)
+b.step(1)
+assert count("malloc") > 0 and any("k_batch_sweepIdLi4E" in k for k in launches())
+b.remove(c)
+c.step(4)
+assert "k_block_stepsIdLi0E" in launches()[-1]
+""")
