@@ -1,6 +1,8 @@
 """Staged transfers over the sizes at which their chunks change (512 KiB up
 to 16 MiB, 1 MiB up to 64 MiB, 2 MiB beyond; 2 MiB towards the device), and
 with the pinned memory made larger and given back between them."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -44,3 +46,29 @@ def test_the_chunks_of_a_transfer_follow_the_steps_before_it():
             assert np.any(ctx.get("uz")[1:] != a[1:])
     finally:
         ctx.close()
+
+
+def test_threads_of_one_device_all_finish():
+    """Four host threads' transfers and audits over the one pinned piece: each
+    ends, within a minute, with its own values."""
+    ctxs = [_context(700 + 300 * i) for i in range(4)]
+    left = list(range(4))
+
+    def work(i):
+        rng = np.random.default_rng(i)
+        for _ in range(6):
+            a = rng.standard_normal(ctxs[i]._shapes["uy"])
+            ctxs[i].set("uy", a)
+            assert np.isfinite(ctxs[i].energy())
+            assert np.array_equal(ctxs[i].get("uy"), a)
+        left.remove(i)
+
+    threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not any(t.is_alive() for t in threads)
+    assert not left
+    for c in ctxs:
+        c.close()

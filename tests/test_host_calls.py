@@ -208,3 +208,64 @@ b.remove(c)
 c.step(4)
 assert "k_block_stepsIdLi0E" in launches()[-1]
 """)
+
+
+def test_the_quotient_cases_run_quotients(runtime):
+    """test_gpu_quotient_tiles.py's meshes march with quotients; in
+    test_gpu_quotient.py the small ones step in blocks (with divisions), and
+    the one with stiffnesses near 1e-9 is out of the quotients' range and
+    divides."""
+    run(runtime, """
+import test_gpu_quotient_tiles as q
+
+def routed(nodes, h, stiffness, sponge, tile):
+    c = fdtd.Context(q._spec(nodes, h, stiffness, 3, sponge), precision="fp64", kernel="tiled" if tile[0] else "auto",
+                     tile_j=tile[0], tile_z=tile[1])
+    n = len(launches())
+    c.step(3)
+    c.close()
+    return launches()[n]
+
+for nodes, h, stiffness, sponge, tile in q.CASES:
+    k = routed(nodes, h, stiffness, sponge, tile)
+    assert "k_sweep_tiledIdLi4ELb%dE" % sponge in k, (nodes, k)
+    assert tile == (0, 0) or k.count("ELi%dELi%dEE" % tile) == 1, k
+assert "k_block_stepsIdLi0ELb0E" in routed((24, 17, 9), 0.3, 1.0, False, (0, 0))
+assert "k_block_stepsIdLi0ELb1E" in routed((24, 17, 9), 1e-4, 5e10, True, (0, 0))
+assert "k_sweep_tiledIdLi0ELb0E" in routed((70, 66, 70), 0.7, 1e-9, False, (0, 0))
+assert "k_sweep_tiledIdLi4ELb1E" in routed((70, 66, 70), 1e-4, 1e11, True, (0, 0))
+""")
+
+
+def test_the_block_step_cases_step_in_blocks(runtime):
+    """test_gpu_block.py's meshes step in blocks in every precision, between
+    them in launches of 1 to 4 steps and cut along every axis; a mesh beyond
+    the dispatch's line marches."""
+    run(runtime, """
+import test_gpu_block as t
+
+cases = next(m for m in t.test_block_steps_equal_the_per_node_sweep.pytestmark if m.args[0].startswith("nodes")).args[1]
+steps, cut, threads = set(), [0, 0, 0], 0
+for precision in ("fp64", "fp32", "fp32c"):
+    for nodes, h, graded, sponge, surface, every in cases:
+        c = fdtd.Context(t._spec(nodes, h, graded, sponge, surface, every, 23), precision=precision)
+        n = len(launches())
+        for calls in (1, 2, 3, 4, 5, 8):
+            c.step(calls)
+        c.close()
+        done = 0
+        for i in range(n, len(launches())):
+            assert "k_block_steps" in launches()[i], (precision, nodes, launches()[i])
+            b = (ctypes.c_int * 5)()
+            hip.host_blocks(i, b)
+            done += b[3]
+            steps.add(b[3])
+            cut = [max(a, v) for a, v in zip(cut, b)]
+            threads = max(threads, b[4])
+        assert done == 23
+assert steps == {1, 2, 3, 4} and min(cut) > 1 and threads > 512, (steps, cut, threads)
+for precision in ("fp64", "fp32", "fp32c"):
+    c = context((64, 64, 40), precision=precision, tune=True)
+    c.step(1)
+    assert not any("k_block_steps" in k for k in launches()[-2:])
+""")
