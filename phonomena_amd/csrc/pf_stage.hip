@@ -14,12 +14,14 @@ namespace {
 constexpr int MAX_DEVICES = 64;
 
 constexpr int SLOTS = 2 * STAGE_LANES;
+constexpr int GROUPS = 5;  // launches that fill all slots: 1, 1, 2, 4, 8 chunks
 
 struct Device {
     std::mutex use;  // held for a transfer
     char* pinned = nullptr;
     size_t room = 0;
     hipEvent_t done[SLOTS] = {};  // a slot's chunk has been written or read
+    hipEvent_t group[GROUPS] = {};
     std::mutex count;
     int users = 0;  // contexts
 };
@@ -34,8 +36,11 @@ void give_back(Device& d) {
 // At least `bytes` of pinned memory, and the events.
 hipError_t reserve(Device& d, size_t bytes) {
     hipError_t e = hipSuccess;
-    for (hipEvent_t& v : d.done)
+    auto make = [&](hipEvent_t& v) {
         if (!v && e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+    };
+    for (hipEvent_t& v : d.done) make(v);
+    for (hipEvent_t& v : d.group) make(v);
     if (e != hipSuccess || d.room >= bytes) return e;
     give_back(d);
     e = hipHostMalloc((void**)&d.pinned, bytes, hipHostMallocDefault);
@@ -122,13 +127,19 @@ int stage_out(int dev, hipStream_t after, void* host, size_t bytes, const StageF
     const Ring r = ring_of(dev, bytes, chunk, lock);
     *taken = r.d != nullptr;
     if (!r.d || !bytes) return PF_OK;
-    auto issue = [&](size_t c) {
-        const hipError_t e = fill(after, r.at(c), c * chunk, r.len(c));
-        return e != hipSuccess || r.chunks == 1 ? e : hipEventRecord(r.done(c), after);
-    };
-    // a chunk for every lane before the threads start
+    const Device& st = *r.d;
+    // every slot's first chunk before the threads start, in groups that grow:
+    // the first copy starts soon, and the gaps between launches stay few
+    const size_t first = r.chunks < (size_t)(2 * r.lanes) ? r.chunks : (size_t)(2 * r.lanes);
+    hipEvent_t ready[SLOTS];
     hipError_t e = hipSuccess;
-    for (int w = 0; w < r.lanes && e == hipSuccess; w++) e = issue((size_t)w);
+    for (size_t c = 0, g = 0; c < first && e == hipSuccess; g++) {
+        size_t n = c < 2 ? 1 : c;
+        if (n > first - c) n = first - c;
+        e = fill(after, r.at(c), c * chunk, (n - 1) * chunk + r.len(c + n - 1));
+        if (e == hipSuccess && r.chunks > 1) e = hipEventRecord(st.group[g], after);
+        while (n--) ready[c++] = st.group[g];
+    }
     if (r.chunks == 1) {
         if (e == hipSuccess) e = hipStreamSynchronize(after);
         if (e == hipSuccess) memcpy(host, r.at(0), bytes);
@@ -136,9 +147,11 @@ int stage_out(int dev, hipStream_t after, void* host, size_t bytes, const StageF
         e = on_lanes(dev, r.lanes, [&](int w) {
             hipError_t v = hipSuccess;
             for (size_t c = (size_t)w; c < r.chunks && v == hipSuccess; c += (size_t)r.lanes) {
-                if (c + (size_t)r.lanes < r.chunks) v = issue(c + (size_t)r.lanes);
-                if (v == hipSuccess) v = hipEventSynchronize(r.done(c));
+                v = hipEventSynchronize(c < first ? ready[c] : r.done(c));
                 if (v == hipSuccess) memcpy((char*)host + c * chunk, r.at(c), r.len(c));
+                const size_t next = c + (size_t)(2 * r.lanes);  // into the slot just read
+                if (v == hipSuccess && next < r.chunks) v = fill(after, r.at(next), next * chunk, r.len(next));
+                if (v == hipSuccess && next < r.chunks) v = hipEventRecord(r.done(next), after);
             }
             return v;
         });

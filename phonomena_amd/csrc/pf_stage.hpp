@@ -13,7 +13,9 @@
 // GB) take 35 ms (46 GB/s) against 154; 1.6 MB of a small mesh's fields 0.2
 // against 0.27.  Chunks of 512 KiB to 2 MiB by the size: a larger one costs
 // fewer launches (of about 6 us beside a chunk's PCIe time), smaller ones keep
-// the lanes of a short transfer busy.
+// the lanes of a short transfer busy; the first two chunks of every lane are
+// filled by five launches (three fields of 9 MB 1.40 ms, with a launch for
+// each 1.47).
 //
 // The lanes have no streams of their own.  With one each the kernels of
 // several chunks overlapped, and 512 KiB chunks were as fast (37 ms there),
@@ -26,11 +28,11 @@
 //
 // The pinned memory of a device is one piece, of 512 KiB with its first
 // context and made again when a transfer needs a larger one (two chunks a
-// lane: 32 MiB at most; 8 MiB take 45 us).  It is shared by every context on the device and stays
-// between calls; when the device's last context is destroyed a piece of more
-// than STAGE_KEEP is given back (a program of many short runs would make a
-// smaller one again for each), and pf_trim gives back all.  A transfer that
-// finds it taken (another host thread's) copies directly.
+// lane: 32 MiB at most; 8 MiB take 45 us).  It is shared by every context on
+// the device and stays between calls; when the device's last context is
+// destroyed a piece of more than STAGE_KEEP is given back (a program of many
+// short runs would make a smaller one again for each), and pf_trim gives back
+// all.  A transfer that finds it taken (another host thread's) copies directly.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -1,5 +1,6 @@
 """Staged transfers over the sizes at which their chunks change (512 KiB up
-to 16 MiB, 1 MiB up to 64 MiB, 2 MiB beyond; 2 MiB towards the device), and
+to 16 MiB, 1 MiB up to 64 MiB, 2 MiB beyond; 2 MiB towards the device) and
+at which the first of them are issued in one more group, and
 with the pinned memory made larger and given back between them."""
 import threading
 
@@ -20,7 +21,8 @@ def _context(nx):
                         precision="fp64", tune=False)
 
 
-@pytest.mark.parametrize("planes", [(255, 2048, 8193), (8192,), (2049, 256), (4097, 64)])
+@pytest.mark.parametrize("planes", [(255, 2048, 8193), (8192,), (2049, 256), (4097, 64),
+                                    (128, 130, 192, 300, 576, 1024, 1025, 1088)])  # 2, 3, 5, 9, 16, 17 chunks
 def test_round_trips_where_the_chunks_change(planes):
     for n in planes:
         ctx = _context(n + 1)
