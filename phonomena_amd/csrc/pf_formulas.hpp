@@ -184,8 +184,8 @@ PF_DEV R div3_uz_surface(R d1, R g1, R d2, R g2, R t3k1, R t3k0, R fz0) {
 // u_new = 2 u - u_old + coef * div (base_solver.py:441-443).  In FP32 the
 // difference takes one fused operation (2 u is exact, and where it would
 // overflow a difference that does not is kept); in FP64 two, since 2 u
-// overflows there in the reference (fused it measured no faster).  With a damping
-// term s > 0 (sponge extension): ((2u - (1-s) u_old) + coef*div) / (1+s);
+// overflows there in the reference (fused it measured no faster).  With a
+// damping term s > 0 (sponge extension): ((2u - (1-s) u_old) + coef*div) / (1+s);
 // in FP32 the division is a product with the hardware reciprocal of 1+s
 // (v_rcp_f32, within 1 ulp; one per node, shared by its three components:
 // the same expression in every call, so the compiler forms it once), where
@@ -276,7 +276,7 @@ PF_DEV void leap_comp(float hi, float lo, float ohi, float olo, float f, float s
         float r = __builtin_amdgcn_rcpf(1.0f + s);  // as in leap()
         float h2 = nh * r;
         float l2 = mad(nh, r, -h2) + nl * r;
-        // |nl| <= ulp(nh) / 2 and r > 1 / 2: |l2| < 2 ulp(h2) <= |h2|
+        // |nl r| <= ulp(nh) r / 2 <= ulp(h2): |l2| < 2 ulp(h2) <= |h2|
         fast_two_sum(h2, l2, nhi, nlo);
     }
 }

@@ -1,5 +1,5 @@
 // Device side of the FDTD step: mesh view, stress/displacement stencils, the
-// naive sweep, the boundary-face kernel, probes, energy audit, pack/unpack.
+// naive sweep, the boundary-face kernel with the probes, pack/unpack.
 //
 // Layout in HBM (one mesh): each displacement component is a dense
 // (nx, ny, pz) array, z contiguous, row stride pz (= nz: unpadded), for two
@@ -637,14 +637,6 @@ __global__ __launch_bounds__(256) void k_sweep_naive(Mesh<R> m) {
     const long long tt = step_index(m);
     if (tt >= m.nsteps) return;
     naive_cell<R, MODE, SPONGE>(m, i, j, k, (R)m.wave[tt]);
-}
-
-// Tiny kernel: advance a device step counter after a captured chunk.
-static __global__ void k_advance(long long* counter, long long by, long long cap) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        long long v = *counter + by;
-        *counter = v < cap ? v : cap;
-    }
 }
 
 // ------------------------------------------------------- pack/unpack ----

@@ -43,10 +43,11 @@
 //
 // Measured, the whole call with Hann window and the first half of the
 // frequencies (before: radix-2 passes, M >= 2n - 1, tables made on the host
-// on each call, a device allocation per array): 1024 traces of 5000 values
-// 6.4 ms (15.8), 64 of 50,000 3.3 (12.0), 8 of 400,000 3.5 (16.1), one of 5000
-// 0.13 (0.57); what is left is the pageable copies over PCIe.  The error
-// against 64 bits went from 9e-16 to 6e-16 (relative 2-norm).
+// on each call, a device allocation per array, pageable copies): 1024 traces
+// of 5000 values 3.0 ms (15.8), 64 of 50,000 2.3 (12.0), 8 of 400,000 2.5
+// (16.1), one of 5000 0.10 (0.57).  Of the first, 6.4 with pageable copies,
+// the kernels are 0.4 and the two staged copies (pf_stage.hpp) the rest.  The
+// error against 64 bits went from 9e-16 to 6e-16 (relative 2-norm).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -83,8 +83,9 @@ def test_fp64_crystal_two_materials():
 def test_fp64_spacings_bitwise_vs_oracle(spacing, sponge):
     """On power-of-two spacings the FP64 tiled sweep takes each division by
     a spacing as a product with its exact reciprocal; on any other spacing it
-    divides.  Both must give the oracle's bits (which divides), on every
-    tile shape and with or without the absorbing layer."""
+    takes exact quotients from reciprocals, or divides where displacements
+    are out of their range.  All must give the oracle's bits (which divides),
+    on every tile shape and with or without the absorbing layer."""
     cells = (36, 30, 20)
     _, _, _, ids, rows, dt, wave = uniform_crystal(
         cells, min(spacing), incl=(19300.0, 2.0e11, 1.6e11, 12, 4), steps=160, seed=5)

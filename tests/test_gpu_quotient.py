@@ -1,8 +1,10 @@
-"""FP64 quotients from reciprocals (the tiled sweep and block steps on
-spacings that are not powers of two) against the per-node sweep, which
-divides: the same bits over the displacements' whole range, where a block
-falls back to divisions (tiny and huge values, zeros among them) and where
-it does not, on blocks, interior tiles and tiles at every face."""
+"""FP64 on spacings that are not powers of two against the per-node sweep,
+which divides: the same bits over the displacements' whole range.  The tiled
+sweep takes quotients from reciprocals where stiffnesses are within their
+range, and a tile falls back to divisions for tiny and huge values, zeros
+among them (the mesh with a layer here; interior tiles without one in
+test_gpu_quotient_tiles.py); block steps, and the tiled sweep at stiffnesses
+out of the range, divide."""
 import numpy as np
 import pytest
 
@@ -49,7 +51,7 @@ def _start(nodes, kind, seed=3):
 @pytest.mark.parametrize("nodes,h,stiffness,sponge", [
     ((24, 17, 9), 0.3, 1.0, False),         # block steps
     ((24, 17, 9), 1e-4, 5e10, True),
-    ((70, 66, 70), 0.7, 1e-9, False),       # the march: 8 x 32 tiles, interior and at every face
+    ((70, 66, 70), 0.7, 1e-9, False),       # the march, dividing: stiffnesses below the quotients' range
     ((70, 66, 70), 1e-4, 1e11, True),
 ])
 @pytest.mark.parametrize("kind", ["full", "decay", "spots"])
