@@ -598,20 +598,14 @@ template <class K> int blocks_per_cu(K kernel, int threads) {
 
 // Planes per x chunk, from the rounds in which the device runs the blocks.
 // per tiles per plane, each block marching xc planes plus `warm` planes it
-// only loads and computes, in pairs, after a start that costs about `start`
-// planes; `slots` blocks resident at once.  Over the balanced chunkings (n
-// chunks of ceil(nx / n) planes, lo <= planes <= cap) the one with the most
-// useful planes per resident-block plane time:
-//     per * nx / (slots * rounds * (even(xc + warm) + start)),
-//     rounds = ceil(per * n / slots)
+// only loads and computes; `slots` blocks resident at once.  Over the
+// balanced chunkings (n chunks of ceil(nx / n) planes, lo <= planes <= cap)
+// the one with the most useful planes per resident-block plane time:
+//     per * nx / (slots * rounds * (xc + warm)),  rounds = ceil(per * n / slots)
 // which charges a last round that leaves CUs idle and the warm-up planes
-// of short chunks.  Ties go to more chunks.  The one-step sweep takes chunks
-// down to 2 planes: where a launch is one round (meshes under about a
-// million nodes) its time is the planes a block marches one after another
-// (0.7 us each in FP32, 1.6 us in FP64 with divisions).  Measured against
-// chunks of at least 16 planes, microseconds a step: 65 x 65 x 33 nodes FP32
-// 12.7 / 22.8, FP32C 18.1 / 37.5, FP64 18.9 / 39.4; 58 x 39 x 13 FP64 15.8 /
-// 45.5; 129 x 129 x 65 FP32 21.3 / 25.9, FP32C 34.4 / 41.4.
+// of short chunks.  With start > 0 a block's planes are counted in the pairs
+// the march runs, after a start that costs about `start` of them:
+// even(xc + warm) + start.  Ties go to more chunks.
 inline int round_xchunk(long long per, int nx, int warm, int start, int lo, int cap, long long slots) {
     int best = nx < cap ? nx : cap;
     double best_s = -1.0;
@@ -623,7 +617,7 @@ inline int round_xchunk(long long per, int nx, int warm, int start, int lo, int 
         if (nc != n) continue;  // same chunking as a smaller n
         const long long blocks = per * nc;
         const long long rounds = (blocks + slots - 1) / slots;
-        const int planes = (xc + warm + 1) / 2 * 2 + start;
+        const int planes = start ? (xc + warm + 1) / 2 * 2 + start : xc + warm;
         const double sc = (double)per * nx / ((double)slots * (double)rounds * (double)planes);
         if (sc >= best_s) {
             best_s = sc;
@@ -633,7 +627,23 @@ inline int round_xchunk(long long per, int nx, int warm, int start, int lo, int 
     return best;
 }
 
-// slots > 0: x chunks by round_xchunk for that many resident blocks;
+// Planes per x chunk of the one-step sweep: at least 16, unless those chunks
+// run in one round.  Then a launch's time is the planes a block marches one
+// after another (0.7 us each in FP32, 1.6 us in FP64 with divisions) and chunks
+// go down to 2 planes, with the start charged.  Measured, short / at least 16
+// planes, us a step: 65 x 65 x 33 nodes FP32 12.7 / 22.8, FP32C 18.1 / 37.5,
+// FP64 18.9 / 39.4; 58 x 39 x 13 FP64 15.8 / 45.5; 129 x 129 x 65 FP32 18.7 /
+// 23.8, FP32C 29.9 / 36.7, FP64 30.6 / 35.1; 225 x 225 x 113 FP32C 80 / 87.
+// Over several rounds the start charge takes long chunks, which lose: 193 x 193
+// x 97 FP64 77.4 / 74.4, 450 x 400 x 200 FP64 630 / 601 and 752 / 705 (with
+// quotients), 513 x 513 x 257 FP32 626 / 594, FP32C 976 / 953, FP64 1133 / 1112.
+inline int sweep_xchunk(long long per, int nx, long long slots) {
+    const int xc = round_xchunk(per, nx, 1, 0, 16, XT - 3, slots);
+    if (per * ((nx + xc - 1) / xc) > slots) return xc;
+    return round_xchunk(per, nx, 1, 2, 2, XT - 3, slots);
+}
+
+// slots > 0: x chunks by sweep_xchunk for that many resident blocks;
 // otherwise a fixed rule.  An explicit xchunk > 0 is kept (within range).
 inline TileMap tile_map(const pf_ctx* c, int tj, int kz, int xchunk, long long slots = 0) {
     TileMap tm;
@@ -643,7 +653,7 @@ inline TileMap tile_map(const pf_ctx* c, int tj, int kz, int xchunk, long long s
         // chosen once per shape: the search costs as much host time as a launch
         auto& a = c->auto_chunk;
         if (a.tj != tj || a.kz != kz || a.slots != slots)
-            a = {tj, kz, slots, round_xchunk((long long)tm.nkt * tm.njt, c->nx, 1, 2, 2, XT - 3, slots)};
+            a = {tj, kz, slots, sweep_xchunk((long long)tm.nkt * tm.njt, c->nx, slots)};
         xchunk = a.xchunk;
     } else if (xchunk <= 0) {
         // aim for >= ~2048 blocks (8 per CU) with chunks of at least 16 planes

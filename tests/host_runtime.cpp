@@ -30,8 +30,10 @@ static std::vector<std::string> g_launches;
 static std::atomic<int> g_fail_host_malloc{0}, g_fail_new{0};
 static std::atomic<int> g_marks{0};
 static float (*g_elapsed)(int, int) = nullptr;
-struct Blocks { int ntx, nty, ntz, steps, threads; };  // a block-step launch's partition (its eighth argument)
-static std::vector<Blocks> g_blocks;
+// a block-step launch's partition (its eighth argument: boxes along x, y, z,
+// steps, threads), a one-step sweep's tiles (its second: along z, y, x, planes)
+struct Grid { int v[5]; };
+static std::vector<Grid> g_grids;
 struct Call { Dim3 grid, block; size_t lds; Stream* stream; };
 static thread_local Call t_call;
 
@@ -58,7 +60,7 @@ long long host_count(const char* what) {
 }
 int host_launches() { return (int)g_launches.size(); }
 const char* host_launch(int i) { return g_launches[(size_t)i].c_str(); }
-void host_blocks(int i, int* out) { memcpy(out, &g_blocks[(size_t)i], sizeof(Blocks)); }
+void host_grid(int i, int* out) { memcpy(out, &g_grids[(size_t)i], sizeof(Grid)); }
 void host_fail_host_malloc(int on) { g_fail_host_malloc = on; }
 void host_fail_new(int on) { g_fail_new = on; }
 void host_elapsed(float (*f)(int, int)) { g_elapsed = f; }
@@ -162,8 +164,9 @@ hipError_t hipLaunchKernel(const void* f, Dim3, Dim3, void** args, size_t lds, S
     if (lds > 65536) count("large_lds", dev);
     std::lock_guard<std::mutex> l(g_lock);
     g_launches.push_back(g_names[f]);
-    g_blocks.push_back({});
-    if (g_names[f].find("k_block_steps") != std::string::npos) memcpy(&g_blocks.back(), args[7], sizeof(Blocks));
+    g_grids.push_back({});
+    if (g_names[f].find("k_block_steps") != std::string::npos) memcpy(&g_grids.back(), args[7], 5 * sizeof(int));
+    if (g_names[f].find("k_sweep_tiled") != std::string::npos) memcpy(&g_grids.back(), args[1], 4 * sizeof(int));
     auto room = g_lds.find({f, dev});
     if ((long long)lds > (room == g_lds.end() ? 65536 : room->second)) return t_error = 1;
     return 0;

@@ -27,6 +27,11 @@ def count(what):
 def launches():
     return [hip.host_launch(i).decode() for i in range(hip.host_launches())]
 
+def grid(i):
+    v = (ctypes.c_int * 5)()
+    hip.host_grid(i, v)
+    return list(v)
+
 def device():
     d = ctypes.c_int()
     hip.hipGetDevice(ctypes.byref(d))
@@ -256,8 +261,7 @@ for precision in ("fp64", "fp32", "fp32c"):
         done = 0
         for i in range(n, len(launches())):
             assert "k_block_steps" in launches()[i], (precision, nodes, launches()[i])
-            b = (ctypes.c_int * 5)()
-            hip.host_blocks(i, b)
+            b = grid(i)
             done += b[3]
             steps.add(b[3])
             cut = [max(a, v) for a, v in zip(cut, b)]
@@ -269,3 +273,34 @@ for precision in ("fp64", "fp32", "fp32c"):
     c.step(1)
     assert not any("k_block_steps" in k for k in launches()[-2:])
 """)
+
+
+@pytest.mark.parametrize("cells,tile,rounds", [
+    ((60, 60, 60), (16, 64), 1), ((60, 60, 60), (8, 32), 1), ((128, 128, 28), (8, 32), 1),
+    ((257, 795, 11), (16, 64), 2), ((136, 614, 11), (8, 32), 2), ((166, 515, 11), (8, 32), 2)])
+def test_x_chunks_by_the_rounds_of_a_launch(runtime, cells, tile, rounds):
+    """A launch of several rounds takes the chunk of at least 16 planes with the
+    most useful planes per plane time; one that is a single round with such
+    chunks may take shorter ones."""
+    run(runtime, """
+cells, tile = %r, %r
+slots = 2 * 256  # the stand-in's resident blocks
+c = context(cells, precision="fp32", kernel="tiled", steps=2)
+c = fdtd.Context(c.spec, precision="fp32", kernel="tiled", tile_j=tile[0], tile_z=tile[1])
+c.step(1)
+i = max(i for i, k in enumerate(launches()) if "k_sweep_tiled" in k)
+nz, ny, nx, planes = grid(i)[:4]
+n = cells[0] + 1
+assert nx == -(-n // planes)
+useful = {}
+for k in range(1, n + 1):
+    p = -(-n // k)
+    if 16 <= p <= 253 and -(-n // p) == k:
+        useful[p] = n / (-(-(ny * nz * k) // slots) * (p + 1))
+best = max(useful.values())
+long = min(p for p in useful if useful[p] == best)  # ties: more chunks
+if ny * nz * -(-n // long) > slots:
+    assert %d > 1 and planes == long, (planes, long)
+else:
+    assert %d == 1 and ny * nz * nx <= slots and planes <= long, (planes, long)
+""" % (cells, tile, rounds, rounds))
