@@ -85,7 +85,16 @@ template <class H, class R> PF_DEV H spacing(R h, R y) {
 // sweep with quotients, with divisions: 205 x 193 x 101 nodes 101 us, 118; with
 // an absorbing layer 121, 129; 257 x 257 x 129 with one 235, 250; 129 x 129 x
 // 65 with one 46, 54.  Noting the range costs 8 of the 101; a second
-// correction, which needs no check of the spacings, 10.
+// correction, which needs no check of the spacings, 10.  Where every tile is
+// out of range the same mesh takes 146 us: the divisions of that branch cost
+// more than in a kernel that only divides.  Displacements below 2^-752 are the
+// tail ahead of a first wave.  With c dt / h = 0.5 it is short, and the first
+// 150 to 1200 steps from rest run as the rest do (100 us, 119); with 0.17 it
+// fills part of the mesh for some hundred steps, and they take 106, 123, 127
+// and 113 us a step over the first 150, 300, 600 and 1200, against 119.  A byte
+// per tile that keeps a tile dividing, a look at the dividends themselves and
+// a copy of the whole step for each flavour cost the near case more (124, 103
+// and spilled registers).
 PF_DEV double quotient(double a, Div<double> d) {
     const double q = a * d.y;
     return __builtin_fma(__builtin_fma(-d.h, q, a), d.y, q);
